@@ -12,8 +12,8 @@
 // F32 per query vector. Blocks of at most 16 vectors (decode rows) let the four waves
 // interleave 32-key tiles and merge through LDS; larger blocks give each wave 16 vectors.
 //
-// F32 KV (F32 execution) or other head dims: the F32 VALU kernel, one work item per
-// (row, KV head, split), one thread per key for the scores and coalesced value reads.
+// F32 KV (F32 execution) or other head dims: the F32 VALU kernel, one workgroup per
+// (row, KV head, split).
 //
 // Splits of one query block are merged by the combine kernel. Scores, softmax and
 // accumulation are F32 (cpp/src/cpu/llama.cpp:67-112; cpp/src/cuda/stage.cpp:291-300).
@@ -24,19 +24,12 @@
 namespace hllm_rocm {
 namespace {
 
-
 constexpr int kThreads = 256;
-constexpr int kTile = 256;
-constexpr int kMaxPairs = 8;  // (head, dim) pairs per thread: G * D <= 2048
 
 __device__ inline floatx4 mfma(half8 a, half8 b, floatx4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
 }
 
-__device__ inline float wave_max(float v) {
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-  return v;
-}
 __device__ inline float wave_sum(float v) {
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
   return v;
@@ -57,6 +50,16 @@ __device__ inline float* partial_at(const AttentionArgs& a, int row, int qh, int
 
 template <int E, bool kCoherent>
 __device__ inline void merge_splits(const AttentionArgs& a, int r, int qh, int splits, int lane);
+
+// Zeroes the operand's padded columns of row r (their weights are zero; the values must be
+// finite) with `threads` threads.
+__device__ inline void zero_padding(const AttentionArgs& a, int r, int thread, int threads) {
+  for (uint64_t c = (uint64_t)a.q_heads * a.head_dim + thread; c < a.out_cols_padded; c += threads) {
+    const uint64_t at = flayout_index(r, c, a.out_cols_padded);
+    a.out_hi[at] = 0;
+    if (a.out_lo) a.out_lo[at] = 0;
+  }
+}
 
 // ---------------------------------------------------------------- MFMA flash attention
 
@@ -639,114 +642,194 @@ __global__ void __launch_bounds__(kThreads, D <= 128 ? 3 : 1) attention_mfma_ker
 
 // ---------------------------------------------------------------- F32 VALU attention
 
+// Keys per split of a row of `ctx` keys: whole 32-key tiles.
 __device__ inline int valu_split_length(int ctx, int max_splits, int unit) {
   int splits = (ctx + unit - 1) / unit;
   splits = splits < max_splits ? splits : max_splits;
   const int per = (ctx + splits - 1) / splits;
-  return (per + 15) & ~15;
+  return (per + 31) & ~31;
 }
 
 template <typename KV>
-__global__ void __launch_bounds__(kThreads) attention_valu_kernel(AttentionArgs a) {
-  const int r = blockIdx.x, kvh = blockIdx.y, s = blockIdx.z;
-  const int ctx = a.row_position[r] + 1;
+__device__ inline floatx4 load4(const KV* p) {
+  if constexpr (sizeof(KV) == 4) {
+    return *reinterpret_cast<const floatx4*>(p);
+  } else {
+    const half4 h = *reinterpret_cast<const half4*>(p);
+    return floatx4{(float)h[0], (float)h[1], (float)h[2], (float)h[3]};
+  }
+}
+
+// Row (r, KV head, split) against HG of the KV head's query heads, F32 arithmetic. Latency-
+// and load-bound: the four waves take interleaved 32-key tiles with an online softmax each
+// (no workgroup barrier until the final merge), and every K/V load is a 16-byte load of
+// consecutive bytes: a key row by LPK lanes of DPL dimensions each (the scores are summed
+// across them), a value row of 32 positions by eight lanes of four positions (summed across
+// them once, after the last tile). A lane-per-key layout read each key row at a stride of D
+// elements and each value one element at a time: 191 -> 28 us per layer for 13 decode rows and
+// an 83-token prompt, Qwen3-0.6B heads. A row whose keys are not split is written here.
+template <typename KV, int D, int HG>
+__global__ void __launch_bounds__(kThreads) attention_valu_kernel(AttentionArgs a, int groups) {
+  constexpr int LPK = D >= 64 ? 16 : D / 4;            // lanes per key
+  constexpr int DPL = D / LPK;                         // dimensions per lane
+  constexpr int KPS = 64 / LPK < 32 ? 64 / LPK : 32;   // keys per step
+  constexpr int STEPS = 32 / KPS;
+  constexpr int DR = D >= 8 ? D / 8 : 1;               // value rows per lane
+  // Steps of keys and rows of values held at once: 32 and 64 registers at D >= 128, so that
+  // three waves share a SIMD (a whole tile's K and V at once left room for two: 38 us).
+  constexpr int SB = STEPS * DPL > 32 ? 32 / DPL : STEPS;
+  constexpr int VB = DR < 16 ? DR : 16;
+  constexpr int kWaves = kThreads / 64;
+  __shared__ __attribute__((aligned(16))) float sc[kWaves][HG][32];
+  __shared__ float merge[kWaves][HG][D + 2];
+  const int r = blockIdx.x, kvh = blockIdx.y / groups, g0 = (blockIdx.y - kvh * groups) * HG, s = blockIdx.z;
+  const int ctx = uniform_load(a.row_position + r) + 1;
   const int per = valu_split_length(ctx, a.max_splits, a.split_unit);
+  const int splits = (ctx + per - 1) / per;
   const int p0 = s * per;
   if (p0 >= ctx) return;
   const int p1 = min(ctx, p0 + per);
-  const int D = a.head_dim, G = a.q_heads / a.kv_heads;
-  const int seq = a.items[a.row_item[r]].sequence;
+  const int G = a.q_heads / a.kv_heads;
+  const int seq = uniform_load(&a.items[uniform_load(a.row_item + r)].sequence);
   const int32_t* table = a.block_table + (size_t)seq * a.table_width;
   const KV* pool = static_cast<const KV*>(a.kv.pool);
   const int bt = a.kv.block_tokens;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int key_lane = (lane / LPK) % KPS, dim0 = (lane % LPK) * DPL;
+  const int quad = lane & 7, row8 = lane >> 3;  // value loads: positions 4 quad .. + 3, row row8 (mod D)
 
-  extern __shared__ float smem[];
-  float* qs = smem;                 // [G][D]
-  float* sc = qs + G * D;           // [G][kTile]
-  float* stat = sc + G * kTile;     // [G] tile max, [G] tile sum
-  const int tid = threadIdx.x;
-  for (int e = tid; e < G * D; e += kThreads) qs[e] = a.q[((size_t)r * a.q_heads + kvh * G) * D + e];
-  const int my_d = tid % D;
-  const int h_first = tid / D, h_step = kThreads / D > 0 ? kThreads / D : 1;
-  float acc[kMaxPairs], run_max[kMaxPairs], run_sum[kMaxPairs];
+  // Heads past the KV head's last repeat it and are not written.
+  float q[HG][DPL], acc[DR][HG], m[HG], l[HG];
 #pragma unroll
-  for (int k = 0; k < kMaxPairs; ++k) {
-    acc[k] = 0.0f;
-    run_max[k] = -INFINITY;
-    run_sum[k] = 0.0f;
+  for (int g = 0; g < HG; ++g) {
+    const float* src = a.q + ((size_t)r * a.q_heads + kvh * G + min(g0 + g, G - 1)) * D + dim0;
+#pragma unroll
+    for (int j = 0; j < DPL; j += 4) {
+      const floatx4 x = *reinterpret_cast<const floatx4*>(src + j);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) q[g][j + i] = x[i];
+    }
+    m[g] = -INFINITY;
+    l[g] = 0.0f;
+#pragma unroll
+    for (int j = 0; j < DR; ++j) acc[j][g] = 0.0f;
+  }
+  for (int t = p0 + 32 * wave; t < p1; t += 32 * kWaves) {
+    const uint64_t block = (uint64_t)uniform_load(table + t / bt);
+    const KV* kb = pool + kv_key_index(a.kv, a.layer, block, t % bt, kvh, 0);
+    const KV* vb = pool + kv_value_index(a.kv, a.layer, block, t % bt, kvh, 0);
+    floatx4 vx[VB];
+    const auto load_values = [&](int j0) {
+#pragma unroll
+      for (int j = 0; j < VB; ++j) vx[j] = load4(vb + (size_t)((8 * (j0 + j) + row8) % D) * 32 + 4 * quad);
+      if (t + 32 > p1) {
+        // Slots past the range hold values no pass has written: a zero probability does not
+        // cancel a non-finite one.
+#pragma unroll
+        for (int j = 0; j < VB; ++j)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (t + 4 * quad + i >= p1) vx[j][i] = 0.0f;
+      }
+    };
+#pragma unroll 1
+    for (int i0 = 0; i0 < STEPS; i0 += SB) {
+      floatx4 kx[SB][DPL / 4];
+#pragma unroll
+      for (int i = 0; i < SB; ++i)
+#pragma unroll
+        for (int j = 0; j < DPL / 4; ++j) kx[i][j] = load4(kb + (size_t)((i0 + i) * KPS + key_lane) * D + dim0 + 4 * j);
+#pragma unroll
+      for (int i = 0; i < SB; ++i) {
+        const int key = (i0 + i) * KPS + key_lane;
+#pragma unroll
+        for (int g = 0; g < HG; ++g) {
+          float dot = 0.0f;
+#pragma unroll
+          for (int j = 0; j < DPL; ++j) dot += q[g][j] * kx[i][j / 4][j % 4];
+#pragma unroll
+          for (int o = 1; o < LPK; o <<= 1) dot += __shfl_xor(dot, o, 64);
+          if (lane % LPK == 0) sc[wave][g][key] = t + key < p1 ? dot * a.scale : -INFINITY;
+        }
+      }
+    }
+    asm volatile("" ::: "memory");  // a wave's LDS accesses complete in order
+    load_values(0);
+    float p[HG][4], alpha[HG];
+#pragma unroll
+    for (int g = 0; g < HG; ++g) {
+      const floatx4 x = *reinterpret_cast<const floatx4*>(&sc[wave][g][4 * quad]);
+      float mx = fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3]));
+#pragma unroll
+      for (int o = 1; o < 8; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+      const float m_new = fmaxf(m[g], mx);
+      alpha[g] = rescale(m[g], m_new);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) p[g][i] = rescale(x[i], m_new);
+      l[g] = l[g] * alpha[g] + ((p[g][0] + p[g][1]) + (p[g][2] + p[g][3]));
+      m[g] = m_new;
+    }
+#pragma unroll
+    for (int j0 = 0; j0 < DR; j0 += VB) {
+      if (j0 > 0) load_values(j0);
+#pragma unroll
+      for (int j = 0; j < VB; ++j)
+#pragma unroll
+        for (int g = 0; g < HG; ++g)
+          acc[j0 + j][g] = acc[j0 + j][g] * alpha[g] +
+                           ((p[g][0] * vx[j][0] + p[g][1] * vx[j][1]) + (p[g][2] * vx[j][2] + p[g][3] * vx[j][3]));
+    }
+    asm volatile("" ::: "memory");
+  }
+#pragma unroll
+  for (int g = 0; g < HG; ++g) {
+#pragma unroll
+    for (int o = 1; o < 8; o <<= 1) {
+      l[g] += __shfl_xor(l[g], o, 64);
+#pragma unroll
+      for (int j = 0; j < DR; ++j) acc[j][g] += __shfl_xor(acc[j][g], o, 64);
+    }
+    if (quad == 0) {
+#pragma unroll
+      for (int j = 0; j < DR; ++j)
+        if (8 * j + row8 < D) merge[wave][g][8 * j + row8] = acc[j][g];
+    }
+    if (lane == 0) {
+      merge[wave][g][D] = m[g];
+      merge[wave][g][D + 1] = l[g];
+    }
   }
   __syncthreads();
-  for (int t0 = p0; t0 < p1; t0 += kTile) {
-    const int n = min(kTile, p1 - t0);
-    if (tid < n) {
-      const int p = t0 + tid;
-      const KV* k = pool + kv_key_index(a.kv, a.layer, (uint64_t)table[p / bt], p % bt, kvh, 0);
-      float dots[8];
+  for (int e = threadIdx.x; e < HG * D; e += kThreads) {
+    const int g = e / D, d = e - g * D;
+    if (g0 + g >= G) continue;
+    const int qh = kvh * G + g0 + g;
+    float mm = -INFINITY;
 #pragma unroll
-      for (int g = 0; g < 8; ++g) dots[g] = 0.0f;
-      for (int d = 0; d < D; ++d) {
-        const float kv = (float)k[d];
+    for (int w = 0; w < kWaves; ++w) mm = fmaxf(mm, merge[w][g][D]);
+    float total = 0.0f, o = 0.0f;
 #pragma unroll
-        for (int g = 0; g < 8; ++g)
-          if (g < G) dots[g] += qs[g * D + d] * kv;
-      }
-#pragma unroll
-      for (int g = 0; g < 8; ++g)
-        if (g < G) sc[g * kTile + tid] = dots[g] * a.scale;
+    for (int w = 0; w < kWaves; ++w) {
+      const float weight = rescale(merge[w][g][D], mm);
+      total += merge[w][g][D + 1] * weight;
+      o += merge[w][g][d] * weight;
     }
-    __syncthreads();
-    const int wave = tid >> 6, lane = tid & 63;
-    for (int g = wave; g < G; g += kThreads / 64) {
-      float mx = -INFINITY;
-      for (int i = lane; i < n; i += 64) mx = fmaxf(mx, sc[g * kTile + i]);
-      mx = wave_max(mx);
-      float sum = 0.0f;
-      for (int i = lane; i < n; i += 64) {
-        const float e = expf(sc[g * kTile + i] - mx);
-        sc[g * kTile + i] = e;
-        sum += e;
+    if (splits > 1) {
+      float* out = partial_at(a, r, qh, s);
+      out[d] = o;
+      if (d == 0) {
+        out[D] = mm;
+        out[D + 1] = total;
       }
-      sum = wave_sum(sum);
-      if (lane == 0) {
-        stat[g] = mx;
-        stat[G + g] = sum;
-      }
+      continue;
     }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < kMaxPairs; ++k) {
-      const int g = h_first + k * h_step;
-      if (tid < G * D && g < G) {
-        const float tile_max = stat[g];
-        const float new_max = fmaxf(run_max[k], tile_max);
-        const float old_scale = rescale(run_max[k], new_max);
-        const float tile_scale = expf(tile_max - new_max);
-        run_sum[k] = run_sum[k] * old_scale + stat[G + g] * tile_scale;
-        run_max[k] = new_max;
-        acc[k] *= old_scale;
-        float part = 0.0f;
-        for (int i = 0; i < n; ++i) {
-          const int p = t0 + i;
-          const KV* v = pool + kv_value_index(a.kv, a.layer, (uint64_t)table[p / bt], p % bt, kvh, my_d);
-          part += sc[g * kTile + i] * (float)*v;
-        }
-        acc[k] += part * tile_scale;
-      }
-    }
-    __syncthreads();
+    const float y = o * (1.0f / total);
+    const uint64_t at = flayout_index(r, (uint64_t)qh * D + d, a.out_cols_padded);
+    const _Float16 hi = to_half(y);
+    a.out_hi[at] = __builtin_bit_cast(uint16_t, hi);
+    if (a.out_lo) a.out_lo[at] = __builtin_bit_cast(uint16_t, to_half((y - (float)hi) * kLoScale));
   }
-#pragma unroll
-  for (int k = 0; k < kMaxPairs; ++k) {
-    const int g = h_first + k * h_step;
-    if (tid < G * D && g < G) {
-      float* out = partial_at(a, r, kvh * G + g, s);
-      out[my_d] = acc[k];
-      if (my_d == 0) {
-        out[D] = run_max[k];
-        out[D + 1] = run_sum[k];
-      }
-    }
-  }
+  if (splits == 1 && kvh == 0 && g0 == 0) zero_padding(a, r, threadIdx.x, kThreads);
 }
 
 // ---------------------------------------------------------------- split combine
@@ -815,18 +898,11 @@ __device__ inline void merge_splits(const AttentionArgs& a, int r, int qh, int s
       if (a.out_lo) a.out_lo[at] = __builtin_bit_cast(uint16_t, to_half((y - (float)hi) * kLoScale));
     }
   }
-  // Zero the operand's padded columns (their weights are zero; the values must be finite).
-  if (qh == 0) {
-    for (uint64_t c = (uint64_t)a.q_heads * D + lane; c < a.out_cols_padded; c += 64) {
-      const uint64_t at = flayout_index(r, c, a.out_cols_padded);
-      a.out_hi[at] = 0;
-      if (a.out_lo) a.out_lo[at] = 0;
-    }
-  }
+  if (qh == 0) zero_padding(a, r, lane, 64);
 }
 
 // One wave per (row, query head), four per block: merge_splits of the row's splits.
-// MFMA-path rows with a single split (or merged by the attention kernel) are skipped.
+// Rows with a single split (or merged by the attention kernel) are skipped.
 template <int E>
 __global__ void __launch_bounds__(256) attention_combine_kernel(AttentionArgs a, int mfma_path) {
   const int pair = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -836,12 +912,12 @@ __global__ void __launch_bounds__(256) attention_combine_kernel(AttentionArgs a,
   int splits;
   if (mfma_path) {
     splits = uniform_load(a.row_splits + r);
-    if (splits == 1) return;
   } else {
     const int ctx = uniform_load(a.row_position + r) + 1;
     const int per = valu_split_length(ctx, a.max_splits, a.split_unit);
     splits = (ctx + per - 1) / per;
   }
+  if (splits == 1) return;
   merge_splits<E, false>(a, r, qh, splits, lane);
 }
 
@@ -860,7 +936,49 @@ void launch_mfma(hipStream_t stream, const AttentionArgs& a) {
            [&] { attention_mfma_kernel<D><<<dim3(a.work_grid * a.kv_heads), kThreads, lds, stream>>>(a); });
 }
 
+// The VALU kernel for the stage's head dim, with the query heads of a KV head in groups of at
+// most HG (a power of two that keeps HG * D / 8 accumulators in registers).
+template <typename KV, int D, int HG>
+void launch_valu_group(hipStream_t stream, const AttentionArgs& a) {
+  const int groups = (a.q_heads / a.kv_heads + HG - 1) / HG;
+  const dim3 grid(a.rows, a.kv_heads * groups, a.work_grid);
+  observed(sizeof(KV) == 4 ? "attention_valu_kernel<float>" : "attention_valu_kernel<_Float16>",
+           [&] { attention_valu_kernel<KV, D, HG><<<grid, kThreads, 0, stream>>>(a, groups); });
+}
+
+template <typename KV, int D>
+void launch_valu_dim(hipStream_t stream, const AttentionArgs& a) {
+  const int G = a.q_heads / a.kv_heads;
+  if (G == 1) return launch_valu_group<KV, D, 1>(stream, a);
+  if (G == 2 || D >= 128) return launch_valu_group<KV, D, 2>(stream, a);
+  if constexpr (D < 128) launch_valu_group<KV, D, 4>(stream, a);
+}
+
+void launch_valu(hipStream_t stream, const AttentionArgs& a) {
+  if (a.kv.f32) {
+    switch (a.head_dim) {
+      case 4: return launch_valu_dim<float, 4>(stream, a);
+      case 8: return launch_valu_dim<float, 8>(stream, a);
+      case 16: return launch_valu_dim<float, 16>(stream, a);
+      case 32: return launch_valu_dim<float, 32>(stream, a);
+      case 64: return launch_valu_dim<float, 64>(stream, a);
+      case 128: return launch_valu_dim<float, 128>(stream, a);
+      case 256: return launch_valu_dim<float, 256>(stream, a);
+    }
+  } else {  // F16 KV at the other head dims runs the MFMA kernel
+    switch (a.head_dim) {
+      case 4: return launch_valu_dim<_Float16, 4>(stream, a);
+      case 8: return launch_valu_dim<_Float16, 8>(stream, a);
+      case 16: return launch_valu_dim<_Float16, 16>(stream, a);
+      case 32: return launch_valu_dim<_Float16, 32>(stream, a);
+    }
+  }
+  fail(HLLM_INTERNAL, "head dimension without an attention kernel");
+}
+
 }  // namespace
+
+int attention_valu_splits(int keys, int max_splits, int unit) { return std::min((keys + unit - 1) / unit, max_splits); }
 
 bool attention_uses_mfma(int head_dim, bool kv_f32) {
   return !kv_f32 && (head_dim == 64 || head_dim == 128 || head_dim == 256);
@@ -876,16 +994,10 @@ void launch_attention(hipStream_t stream, const AttentionArgs& a) {
       if (a.head_dim == 256) launch_mfma<256>(stream, a);
     }
   } else {
-    const int G = a.q_heads / a.kv_heads;
-    const size_t lds = ((size_t)G * a.head_dim + (size_t)G * kTile + 2 * G) * sizeof(float);
-    dim3 grid(a.rows, a.kv_heads, a.max_splits);
-    if (a.kv.f32)
-      observed("attention_valu_kernel<float>", [&] { attention_valu_kernel<float><<<grid, kThreads, lds, stream>>>(a); });
-    else
-      observed("attention_valu_kernel<_Float16>", [&] { attention_valu_kernel<_Float16><<<grid, kThreads, lds, stream>>>(a); });
+    launch_valu(stream, a);
   }
-  // MFMA-path blocks with a single split write their rows directly.
-  if (mfma_path && !a.any_split) return;
+  // Rows with a single split are written by the attention kernel.
+  if (!a.any_split) return;
   const unsigned blocks = (unsigned)(a.rows * a.q_heads + 3) / 4;
   const int path = mfma_path ? 1 : 0;
   observed("attention_combine_kernel", [&] {

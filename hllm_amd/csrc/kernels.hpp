@@ -218,7 +218,7 @@ struct AttentionArgs {
   int rows, q_heads, kv_heads, head_dim;
   const AttnWork* work;        // MFMA path work list, its size (device) and the launch's
   const int32_t* work_count;   // workgroups along x, which loop over the list
-  int work_grid;
+  int work_grid;               // (VALU path: the most key splits of any row)
   int any_split;               // some block's splits are left to the combine kernel
   const int32_t* row_splits;   // [rows] splits the combine kernel merges (1: none)
   int fold;                    // decode-like blocks merge their splits in the attention kernel
@@ -242,6 +242,8 @@ struct AttentionArgs {
 void launch_attention(hipStream_t stream, const AttentionArgs& a);
 // Whether launch_attention uses the MFMA kernel (and hence the pack kernel's work list).
 bool attention_uses_mfma(int head_dim, bool kv_f32);
+// Upper bound of a row's key splits on the VALU path (at least 1; 1 means it is not split).
+int attention_valu_splits(int keys, int max_splits, int unit);
 
 // Row-wise first maximum over `cols` F32 values per row (greedy sampling) and a
 // non-finite flag (bit 1 of flags).

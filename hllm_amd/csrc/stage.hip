@@ -1224,6 +1224,11 @@ void Stage::submit(const hllm_rocm_pass& pass, bool phases) {
                                                 pack_.attn_fold);
     }
     if ((uint64_t)attn_work_count > attn_work_max_) fail(HLLM_INTERNAL, "attention work list overflow");
+  } else {
+    for (uint32_t i = 0; i < n; ++i)
+      attn_work_count = std::max(attn_work_count, attention_valu_splits((int)(pass.item[i].first_position + pass.item[i].query_tokens),
+                                                                        kMaxSplits, kSplitUnit));
+    attn_any_split = attn_work_count > 1;
   }
   // Passes of single-token items (decode rows) at head dim 128 with F16 KV: QK-norm, RoPE and
   // the K/V append run inside the attention kernel (AttentionRope), one launch fewer per layer.
@@ -1235,7 +1240,7 @@ void Stage::submit(const hllm_rocm_pass& pass, bool phases) {
   const int R = (int)rows;
   const int S = (int)sample_items.size();
   // One attention workgroup (per KV head) per work item: the hardware's dispatch balances
-  // items of different lengths.
+  // items of different lengths. VALU path: one per row and split.
   const int attn_grid = attn_work_count;
   // Greedy passes that return no logits take each row's first maximum from the LM head's
   // epilogue (one candidate per workgroup; the logits are never written): its part count,
