@@ -160,9 +160,6 @@ void launch_embed(hipStream_t stream, const uint16_t* table_hi, const uint16_t* 
                   uint64_t cols_padded, const int32_t* row_token, int rows, int hidden, float* h);
 
 void launch_boundary_decode(hipStream_t stream, const uint16_t* in, int rows, int hidden, float* h);
-void launch_boundary_encode(hipStream_t stream, const float* h, int rows, int hidden, uint16_t* out,
-                            int32_t* flags);
-
 // K-split partial outputs a projection left for its consumer: `parts` row-major matrices
 // of the consumer's row width, `stride` floats apart, summed in order (0 = none).
 struct Partials {
@@ -170,6 +167,10 @@ struct Partials {
   int parts = 0;
   uint64_t stride = 0;
 };
+
+// F16 boundary values of h plus its pending partials (flag 4: one is not finite).
+void launch_boundary_encode(hipStream_t stream, const float* h, int rows, int hidden, Partials residual,
+                            uint16_t* out, int32_t* flags);
 
 // y = (x * inv_rms) * w written to F-layout hi (+ lo when lo != nullptr); rows may be
 // gathered through `row_index` (nullptr = identity) with `count` read from device

@@ -1356,11 +1356,10 @@ void Stage::submit(const hllm_rocm_pass& pass, bool phases) {
       });
       gemm("gemm_gate_up", w.gate_up, a0h, a0l, R, (int)(2 * Ip_), kEpiSwiglu, nullptr, 0, a1h, a1l, Ip_);
       // The last layer's down partials are summed by the final norm, for the sampled rows it
-      // gathers (nothing reads the other rows' residual afterwards); a boundary stage sums
-      // them here (the boundary reads the whole stream).
-      const bool defer_down = l + 1 < L_ || c_.final_stage;
+      // gathers (nothing reads the other rows' residual afterwards), or by the boundary's
+      // encoding.
       const int down_parts = gemm("gemm_down", w.down, a1h, a1l, R, (int)H_, kEpiResidual, h, (int)H_, nullptr,
-                                  nullptr, 0, defer_down);
+                                  nullptr, 0, true);
       pending = Partials{ws, down_parts, (uint64_t)R * H_};
       HIP_CHECK(hipGetLastError());
       mark_phase("layer", (int32_t)(c_.layer_start + l));
@@ -1442,7 +1441,7 @@ void Stage::submit(const hllm_rocm_pass& pass, bool phases) {
       }
     } else {
       timed("boundary", (uint64_t)R * H_ * 6, 0.0, [&] {
-        launch_boundary_encode(stream_, h, R, (int)H_, boundary_dev_.as<uint16_t>(), flags_dev());
+        launch_boundary_encode(stream_, h, R, (int)H_, pending, boundary_dev_.as<uint16_t>(), flags_dev());
       });
       HIP_CHECK(hipMemcpyAsync(pin_boundary_.ptr, boundary_dev_.ptr, (size_t)R * H_ * 2, hipMemcpyDeviceToHost,
                                stream_));

@@ -1,0 +1,39 @@
+"""Gate/up projections of few rows (the pair kernel) and the boundary encoding that sums the last
+down projection's K-split partials, against the oracle at their edges: k-steps fewer than the
+waves, not a multiple of them and past one ring; an odd number of 32-feature groups; workgroups
+of one pair and of two (more pairs than CUs); 1 to 64 rows around every 16-row tile; row lengths
+that divide by four and that do not.
+
+A one-layer first stage returns its boundary rows. Bounds per row as for the other F16 slices
+(max-abs 2e-2, cosine 0.9999)."""
+import numpy as np
+import pytest
+
+import oracle
+from hllm_amd import capi, model, synthetic
+from tests import helpers_parity as hp
+from tests import models
+
+pytestmark = pytest.mark.gpu
+ROWS = (1, 15, 16, 17, 31, 33, 48, 49, 64)
+
+
+@pytest.mark.parametrize("hidden,intermediate", [(64, 32), (66, 96), (96, 160), (160, 4128), (544, 288)])
+def test_gate_up_and_boundary_match_the_oracle(hidden, intermediate):
+    shape = synthetic.ModelShape(f"h{hidden}-i{intermediate}", 2, hidden, intermediate, 4, 2, 64, 300, eps=1e-6,
+                                 theta=1e4, qk_norm=False, tied=False, max_seq=128)
+    st = capi.Stage(model.stage_config(shape, 0, 1, first=True, final=False, execution="f16", kv_cache_bytes=16 << 20,
+                                       max_sequences=4, max_pass_rows=128))
+    model.synthesize(st, shape, seed=5, norm_sigma=0.1)
+    ost = oracle.OracleStage(models.synthetic_stage(shape, 0, 1, first=True, final=False, seed=5, norm_sigma=0.1))
+    rng = np.random.default_rng(3)
+    for rows in ROWS:
+        hp.say(shape.name, "rows", rows)
+        ids = rng.integers(0, shape.vocab, rows).astype(np.uint64)
+        seq, oseq = st.allocate(rows), ost.allocate_sequence(rows)
+        got = st.execute([capi.item(seq, rows, 0, sample=False)], token_ids=ids)["boundary"]
+        kind, expect = ost.execute(ids, 0, oseq)[:2]
+        assert kind == "boundary"
+        hp.check_rows(oracle.f16_decode(got), oracle.f16_decode(expect), (shape.name, rows))
+        st.release(seq)
+    st.close()
