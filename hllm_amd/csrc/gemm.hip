@@ -1236,6 +1236,111 @@ __global__ void __launch_bounds__(64 * WAVES) gemm_decode_kernel(GemmArgs a, int
   }
 }
 
+// Gate/up projection of few rows (F16, SwiGLU), HBM- and latency-bound: a workgroup owns NP
+// gate/up pairs of 16 features and its WK waves interleave the k-steps, each streaming its own
+// weight and activation fragments through a ring of P k-steps; the waves' tiles are summed
+// through LDS in wave order. Against the decode kernel's wave per pair this makes WK times as
+// many, shorter streams (every CU has one on narrow models), at the price of reading the
+// activations once per workgroup. Qwen3-0.6B, 12.6 MB of weights: 8.75 -> 5.1 us for one row
+// (1.4 -> 2.5 TB/s), 11.1 -> 6.1 us for 45; 67 MB at K 2 048, seven rows: 17.9 -> 13.9 us
+// (4.8 TB/s). WK 8 and rings of 8 measured the same or up to 1.5 us slower.
+template <int MF, int NP, int WK, int P>
+__global__ void __launch_bounds__(64 * WK) gemm_pair_kernel(GemmArgs a) {
+  constexpr int NF = 2 * NP;
+  extern __shared__ float lds[];  // [WK][MF][NF][64] floatx4
+  const int M = a.device_m ? *a.device_m : a.M;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int KT = (int)(a.Kp >> 5);
+  const size_t frag_stride = (size_t)KT * 64;
+  const int pair0 = blockIdx.x * NP;  // pair p: gate fragment 4 (p / 2) + p % 2, up fragment two further
+  const half8* W[NF];
+#pragma unroll
+  for (int p = 0; p < NP; ++p) {
+    const int gate = 4 * ((pair0 + p) >> 1) + ((pair0 + p) & 1);
+    W[2 * p] = reinterpret_cast<const half8*>(a.w_hi) + (size_t)gate * frag_stride + lane;
+    W[2 * p + 1] = W[2 * p] + 2 * frag_stride;
+  }
+  const half8* X = reinterpret_cast<const half8*>(a.x_hi) + lane;
+  floatx4 acc[MF][NF];
+#pragma unroll
+  for (int i = 0; i < MF; ++i)
+#pragma unroll
+    for (int j = 0; j < NF; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  half8 rb[P][NF], rx[P][MF];
+  const int steps = wave < KT ? (KT - wave + WK - 1) / WK : 0;
+  // Unconditional loads (see gemm_kernel); past the range they re-read the last k-step.
+  auto load = [&](int slot, int step) {
+    const int kt = min(wave + step * WK, KT - 1);
+#pragma unroll
+    for (int i = 0; i < MF; ++i) rx[slot][i] = X[i * frag_stride + (size_t)kt * 64];
+#pragma unroll
+    for (int j = 0; j < NF; ++j) rb[slot][j] = __builtin_nontemporal_load(W[j] + (size_t)kt * 64);
+  };
+  auto compute = [&](int s) {
+#pragma unroll
+    for (int i = 0; i < MF; ++i)
+#pragma unroll
+      for (int j = 0; j < NF; ++j) acc[i][j] = mfma(rb[s][j], rx[s][i], acc[i][j]);
+  };
+#pragma unroll
+  for (int s = 0; s < P; ++s) load(s, s);
+  int base = 0;
+  for (; base + P < steps; base += P) {
+#pragma unroll
+    for (int s = 0; s < P; ++s) {
+      compute(s);
+      load(s, base + s + P);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+#pragma unroll
+  for (int s = 0; s < P; ++s)
+    if (base + s < steps) compute(s);
+
+  floatx4* tiles = reinterpret_cast<floatx4*>(lds);
+#pragma unroll
+  for (int i = 0; i < MF; ++i)
+#pragma unroll
+    for (int j = 0; j < NF; ++j) tiles[((wave * MF + i) * NF + j) * 64 + lane] = acc[i][j];
+  __syncthreads();
+  // Lane (q, t) of pair p holds row 16 i + t, activations 16 (pair0 + p) + 4 q .. + 3.
+  for (int e = threadIdx.x; e < MF * NP * 64; e += 64 * WK) {
+    const int ln = e & 63, p = (e >> 6) % NP, i = (e >> 6) / NP;
+    floatx4 gate = {0.f, 0.f, 0.f, 0.f}, up = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < WK; ++w) {
+      const floatx4 g = tiles[((w * MF + i) * NF + 2 * p) * 64 + ln], u = tiles[((w * MF + i) * NF + 2 * p + 1) * 64 + ln];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        gate[t] += g[t];
+        up[t] += u[t];
+      }
+    }
+    const int row = i * 16 + (ln & 15);
+    const uint64_t col = (uint64_t)(pair0 + p) * 16 + (ln >> 4) * 4;
+    if (row >= M || col >= a.out_cols_padded) continue;
+    half4 vh;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) vh[t] = to_half(silu_mul(gate[t], up[t]));
+    *reinterpret_cast<half4*>(a.out_hi + flayout_index(row, col, a.out_cols_padded)) = vh;
+  }
+}
+
+template <int MF, int NP, int WK, int P>
+void launch_pair_shape(hipStream_t stream, const GemmArgs& a) {
+  if ((uint64_t)MF * 16 > a.x_rows_padded) fail(HLLM_INTERNAL, "GEMM tile exceeds the activation padding");
+  if (a.N % (32 * NP) != 0 || (uint64_t)a.N > a.w_rows_padded) fail(HLLM_INTERNAL, "gate/up pairs exceed the weights");
+  constexpr size_t lds = (size_t)WK * MF * NP * 2 * 1024;
+  static const bool configured = [] {
+    HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_pair_kernel<MF, NP, WK, P>),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    return true;
+  }();
+  (void)configured;
+  observed(kernel_name<MF, NP, WK, P>("gemm_pair_kernel"),
+           [&] { gemm_pair_kernel<MF, NP, WK, P><<<dim3(a.N / (32 * NP)), 64 * WK, lds, stream>>>(a); });
+}
+
 // LDS a decode workgroup may give to its split's whole activation range.
 constexpr size_t kDecodeWholeLds = 144 * 1024;
 namespace {
@@ -1465,6 +1570,16 @@ bool decode_applies(const GemmArgs& a, int prec, int rows, int cus) {
   return n_tiles * waves >= 4 * cus;
 }
 
+// Whether gate/up runs on the pair kernel: up to 16 rows always, more rows where the decode
+// kernel's workgroups (64 pairs' features each) would leave half of the CUs or more without
+// one. Measured per launch (event times), decode kernel -> pair kernel: Qwen3-0.6B (48
+// workgroups) 10.0 -> 6.8 us at 4 rows, 12.4 -> 7.8 at 48, 13.1 -> 8.5 at 64; 16 384 columns of
+// K 2 048 (128) 19.9 -> 15.0 at 4 rows, 21.7 -> 17.4 at 64; Falcon3-3B (144) 25.8 -> 25.3 at 4
+// rows but 25.1 -> 27.8 at 32; Qwen3-4B (152) 21.6 -> 21.0 at 4 and 24.7 -> 30.3 at 64.
+bool pair_applies(const GemmArgs& a, int rows, int cus) {
+  return a.epilogue == kEpiSwiglu && a.N % 64 == 0 && (rows <= 16 || (a.N + 127) / 128 <= cus / 2);
+}
+
 // Fragment rows per wave of the unpaired decode variant: the configured count, halved while
 // the workgroups' tiles would read past the weight rows (padded to 256).
 int decode_frags(const GemmArgs& a, int waves) {
@@ -1492,7 +1607,9 @@ int launch_decode_variant(hipStream_t stream, const GemmArgs& a, int cus) {
     const int per = (chunks + ksplit - 1) / ksplit;
     ksplit = (chunks + per - 1) / per;
   }
-  if (pair) return launch_decode_waves<MF, 2, KC, P, true, P>(stream, a, waves, 1);
+  if constexpr (MF > 1) {  // one row tile: the pair kernel
+    if (pair) return launch_decode_waves<MF, 2, KC, P, true, P>(stream, a, waves, 1);
+  }
   if (nfw == 4) return launch_decode_waves<MF, 4, KC, P, false, (PW > 8 ? 8 : PW)>(stream, a, waves, ksplit);
   if (nfw == 2) return launch_decode_waves<MF, 2, KC, P, false, PW>(stream, a, waves, ksplit);
   return launch_decode_waves<MF, 1, KC, P, false, PW>(stream, a, waves, ksplit);
@@ -1510,7 +1627,29 @@ int launch_decode_rows(hipStream_t stream, const GemmArgs& a, int cus) {
   return launch_decode_variant<MF, 16, 8, 8>(stream, a, cus);
 }
 
+// The pair kernel's shape for passes of at most 16 * MF rows: one pair per workgroup while the
+// workgroups fit the CUs about once, or while one row tile leaves the activations the smaller
+// stream; two above (64 rows, Llama shape of the tests: 17.4 against 20.2 us).
+template <int MF>
+void launch_pair(hipStream_t stream, const GemmArgs& a, int cus) {
+  if constexpr (MF > 1) {
+    if (a.N / 32 > cus) return launch_pair_shape<MF, 2, 4, 4>(stream, a);
+  }
+  launch_pair_shape<MF, 1, 4, 4>(stream, a);
+}
+
 int launch_decode(hipStream_t stream, const GemmArgs& a, int rows, int cus) {
+  if (pair_applies(a, rows, cus)) {
+    if (rows <= 16)
+      launch_pair<1>(stream, a, cus);
+    else if (rows <= 32)
+      launch_pair<2>(stream, a, cus);
+    else if (rows <= 48)
+      launch_pair<3>(stream, a, cus);
+    else
+      launch_pair<4>(stream, a, cus);
+    return 0;
+  }
   if (rows <= 16) return launch_decode_rows<1>(stream, a, cus);
   if (rows <= 32) return launch_decode_rows<2>(stream, a, cus);
   return launch_decode_rows<4>(stream, a, cus);
