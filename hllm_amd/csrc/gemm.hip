@@ -1451,27 +1451,76 @@ struct Choice {
   int ksplit;  // 0: the configuration's own rule
 };
 
+// K splits of a deferred projection for about 280 workgroups of 128 x 256 tiles, at most 8.
+int deferred_splits(int rows, int n, int kt) {
+  const double tiles = (double)((n + 255) / 256) * ((rows + 127) / 128);
+  return std::min({std::max(1, (int)(280.0 / tiles + 0.5)), 8, std::max(1, kt / 8)});
+}
+
+// Tile height and K split of F16 passes of 224 rows and more, by the estimated time: rounds of
+// workgroups over the fullest XCD's CUs (xcd_tile), times the k-steps of a split, times the
+// tile's time per k-step, plus the partials (written here and read back by the consumer, 8
+// bytes per output and split, at about 4.5 TB/s). The times per k-step are those of one round
+// of the Qwen3-4B and Falcon3-3B projections: LDS-copy tiles of 128, 192 and 256 rows 0.51, 0.72
+// and 0.90 us (one workgroup per CU; bound by the copies, so a taller tile is cheaper per
+// row), and activation-staged 128-row tiles 0.8 us with two workgroups per CU (1.0 us in the
+// only round). Measured per layer against the earlier choice by row ranges (all
+// above 768 rows on activation-staged tiles): Falcon3-3B at 1300 rows, q/k/v 77 -> 50, o 45 -> 41,
+// gate+up 164 -> 139, down 112 -> 82 us; Qwen3-4B at 1024 rows 55 -> 44, 42 -> 31, 120 -> 116, 76 ->
+// 54 us; gate+up of Qwen3-0.6B at 512 rows (a K split and a reduce kernel before) 31 -> 23 us.
+Choice tile_choice(int rows, int n, uint64_t kp, bool deferred, size_t workspace_floats, int cus) {
+  struct Tile {
+    int config, bm, per_cu;
+    double step_us, only_round_us;
+  };
+  constexpr Tile kTiles[] = {{15, 128, 1, 0.51, 0.51}, {18, 192, 1, 0.72, 0.72}, {16, 256, 1, 0.90, 0.90},
+                             {9, 128, 2, 0.80, 1.00}};
+  const int n_tiles = (n + 255) / 256, kt = (int)(kp >> 5);
+  const double partial_us = 8.0 * rows * n / 4.5e6;
+  // Above 1536 rows (there the row tiles alone fill the CUs on most shapes) the K split is that
+  // of 280 workgroups of 128-row tiles, as for F32 execution: full passes of long prompts keep
+  // their order of summation, and with it the tokens at near ties, whatever tile runs them.
+  const int kept = rows > 1536 && deferred ? deferred_splits(rows, n, kt) : 0;
+  Choice best{15, 1};
+  double least = 1e30;
+  for (const Tile& t : kTiles) {
+    const int m_tiles = (rows + t.bm - 1) / t.bm, slots = std::max(1, cus / kXcds) * t.per_cu;
+    const int most = kept > 0 ? kept : deferred && t.per_cu == 1 ? 8 : 1;
+    for (int ks = std::max(1, kept); ks <= most; ++ks) {
+      if (ks > 1 && kept == 0 && (kt / ks < 12 || (size_t)ks * rows * n > workspace_floats)) break;
+      const int rounds = ((n_tiles * ks + kXcds - 1) / kXcds * m_tiles + slots - 1) / slots;
+      const double steps_us = (kt + ks - 1) / ks * (rounds == 1 ? t.only_round_us : rounds * t.step_us);
+      const double us = steps_us + (deferred ? ks * partial_us : 0.0);
+      if (us < least) {
+        least = us;
+        best = {t.config, ks};
+      }
+    }
+  }
+  return best;
+}
+
 // Projection configuration by pass rows and shape, from sweeps of the Qwen3 projection
 // shapes on MI355X with weights streamed from HBM:
-//  - up to 64 rows: the register-streaming decode kernels (BM 16/32/64), except for very
-//    wide outputs (gate+up, LM head) with more than 32 rows, where staging the activations
-//    in LDS once per 256-feature tile wins;
-//  - more rows: the activation-staged kernel, BM 64, or BM 128 from 384 rows; wide outputs
-//    from 192 to 768 rows use the kernels that copy both operands to LDS (BM 128 below
-//    448 rows, BM 256 from there), and BM 128 activation-staged tiles beyond; so do the
-//    deferred projections of chunk-sized F16 passes (BM 128, fewer K splits than the
-//    activation-staged kernel needs, so their consumers also read fewer partials).
+//  - up to 64 rows: the register-streaming kernels (BM 16/32/64), except for very wide outputs
+//    (gate+up, LM head) with more than 32 rows, where staging the activations in LDS once per
+//    256-feature tile wins;
+//  - F16 passes from 224 rows: tile_choice;
+//  - the rest: the activation-staged kernel, BM 64, or BM 128 from 384 rows.
 // K is split while there are few output tiles. When the consumer sums the partials
 // (`deferred`) a split costs one partial write, so about 220-280 workgroups are targeted;
 // otherwise a reduce kernel reads every partial back, so splits stop at about 200
 // workgroups, in powers of two.
-Choice gemm_choice(int rows, int n, uint64_t kp, bool deferred, bool f16, int cus) {
+Choice gemm_choice(int rows, int n, uint64_t kp, bool deferred, bool f16, size_t workspace_floats, int cus) {
   const bool wide = n >= 16384;
   const auto rounded = [](double x) { return std::max(1, (int)(x + 0.5)); };
-  if (f16 && deferred && rows > 64 && rows <= 768) {
-    // Deferred projections of chunk-sized F16 passes, with the most K splits whose
-    // workgroups fit every XCD's CUs at once (xcd_tile; one workgroup per CU: a second round
-    // costs up to a third more, q/k/v at 160 rows 18.4 -> 24.1 us).
+  if (f16 && rows >= 224) return tile_choice(rows, n, kp, deferred, workspace_floats, cus);
+  if (f16 && deferred && rows > 64) {
+    // 65-223 rows: 64-row activation-staged tiles (at least two chunks per split), or the
+    // 128-row LDS-copy tiles where they allow more than twice the K splits (less work per
+    // workgroup), with the most K splits whose workgroups fit every XCD's CUs at once
+    // (xcd_tile; a second round costs up to a third more). Measured at 96-208 rows: o 12.0-15.3
+    // us, down 21.5-26.7, q/k/v 13.8-18.3 (24-28 us at 160-208 rows in two rounds).
     const int n_tiles = (n + 255) / 256, per_xcd = std::max(1, cus / kXcds);
     const auto splits = [&](int bm, int least, int most) {
       const int m_tiles = (rows + bm - 1) / bm;
@@ -1479,24 +1528,6 @@ Choice gemm_choice(int rows, int n, uint64_t kp, bool deferred, bool f16, int cu
       while (ks > least && (n_tiles * ks + kXcds - 1) / kXcds * m_tiles > per_xcd) --ks;
       return ks;
     };
-    if (rows >= 224) {
-      // From 224 rows both operands are copied to LDS in 128 x 256 tiles (2 to 8 splits).
-      // Measured on the Qwen3-4B projections against the activation-staged kernel: down 28
-      // against 34-42 us from 288 to 384 rows, q/k/v 20 / 23 against 24 / 27 us at 224 /
-      // 352 rows, o within 1 us. 192 x 256 tiles instead when they allow at least twice the
-      // K splits (a quarter less work per workgroup) and those splits still hold 32 k-steps
-      // or more: down of 513-576-row passes (three row tiles against five), 43.7 -> 37.2 us.
-      // Where 192-row tiles gain less they measured slower (q/k/v at 320-384 rows), and o
-      // (16 k-steps per split) gains 0.6 us while its consumer reads twice the partials.
-      const int ks128 = splits(128, 2, 8), ks192 = splits(192, 2, 8);
-      const bool long_splits = (int)(kp >> 5) / ks192 >= 32;
-      return ks192 >= 2 * ks128 && long_splits ? Choice{18, ks192} : Choice{15, ks128};
-    }
-    // 65-223 rows: 64-row activation-staged tiles (at least two chunks per split), or the
-    // 128-row LDS-copy tiles where they allow more than twice the K splits (less work per
-    // workgroup). Measured at 96-208 rows: o 12.0-15.3 us, down 21.5-26.7, q/k/v 13.8-18.3
-    // (q/k/v at 160-208 rows 24-28 us with the earlier rule of ~280 workgroups, which took
-    // a second round of workgroups on some XCDs).
     const int ks64 = splits(64, 1, std::min(8, std::max(1, (int)(kp >> 5) / 16)));
     const int ks128 = splits(128, 2, 8);
     return 2 * ks64 < ks128 ? Choice{15, ks128} : Choice{12, ks64};
@@ -1507,14 +1538,8 @@ Choice gemm_choice(int rows, int n, uint64_t kp, bool deferred, bool f16, int cu
     const int cap = std::max(1, (int)(kp >> 5) / 8);  // at least two k-steps per K-wave
     return {config, deferred ? std::min(rounded(220.0 / tiles), cap) : 0};
   }
-  if (wide && !deferred && rows > 192 && rows <= 768) {
-    // Both operands copied to LDS, with the tile height that fits the rows in the fewest
-    // rounds of workgroups over the CUs (gate+up of Qwen3-4B, 76 weight tiles: 128-row tiles
-    // up to 384 rows, 192-row tiles (three row tiles, 228 workgroups) up to 576, 256-row
-    // tiles above). Up to 192 rows the activation-staged 64-row tiles fit in one round
-    // (228 workgroups): 35.8 against 45.3 us at 192 rows.
-    return {rows <= 384 ? 15 : rows <= 576 ? 18 : 16, 1};
-  }
+  // Wide outputs of 193-223 rows (and up to 768 in F32 execution): 128-row tiles, unsplit.
+  if (wide && !deferred && rows > 192 && rows <= 768) return {15, 1};
   const int bm = rows >= 384 || (wide && rows > 192) ? 128 : 64;
   const int config = bm == 128 ? 9 : 12;
   const int kc = bm == 128 ? 4 : 8;
@@ -1690,7 +1715,8 @@ int launch_gemm(hipStream_t stream, const GemmArgs& args, int prec, int rows_bou
     return launch_decode(stream, args, rows_bound, cus);
   if (forced == kDecodeConfig && prec == kF16 && rows_bound <= 64 && (args.defer_reduce || args.epilogue == kEpiSwiglu))
     return launch_decode(stream, args, rows_bound, cus);
-  Choice c = gemm_choice(rows_bound, args.N, args.Kp, args.defer_reduce != 0, prec == kF16, cus);
+  Choice c = gemm_choice(rows_bound, args.N, args.Kp, args.defer_reduce != 0, prec == kF16,
+                         args.workspace_floats, cus);
   if (forced >= 0 && forced != kDecodeConfig) c = {forced, 0};
   return launch_gemm_config(stream, args, prec, rows_bound, cus, c.config, c.ksplit);
 }
