@@ -159,6 +159,7 @@ void launch_pack(hipStream_t stream, const ItemMeta* items, int n_items, const i
 void launch_embed(hipStream_t stream, const uint16_t* table_hi, const uint16_t* table_lo,
                   uint64_t cols_padded, const int32_t* row_token, int rows, int hidden, float* h);
 
+// h from F16 boundary values in mapped host memory.
 void launch_boundary_decode(hipStream_t stream, const uint16_t* in, int rows, int hidden, float* h);
 // K-split partial outputs a projection left for its consumer: `parts` row-major matrices
 // of the consumer's row width, `stride` floats apart, summed in order (0 = none).
@@ -168,7 +169,8 @@ struct Partials {
   uint64_t stride = 0;
 };
 
-// F16 boundary values of h plus its pending partials (flag 4: one is not finite).
+// F16 boundary values of h plus its pending partials, written with `flags` (set to 4 when one is
+// not finite) to mapped host memory.
 void launch_boundary_encode(hipStream_t stream, const float* h, int rows, int hidden, Partials residual,
                             uint16_t* out, int32_t* flags);
 

@@ -272,7 +272,7 @@ class Stage {
   // the input tokens; tokens_ the sampled tokens, then the pass's error flags.
   DeviceMemory gemm_ws_, gemm_counters_, logits_, argmax_val_, argmax_idx_, tokens_;
   uint64_t argmax_capacity_ = 0;  // entries of argmax_val_ / argmax_idx_
-  DeviceMemory items_dev_, pack_buf_, boundary_dev_, staging_, attn_work_;
+  DeviceMemory items_dev_, pack_buf_, staging_, attn_work_;
   bool mfma_attention_ = false;
   uint64_t attn_work_max_ = 0;
   size_t gemm_ws_floats_ = 0;
@@ -553,7 +553,6 @@ Stage::Stage(const hllm_rocm_stage_config& c) : c_(c) {
       pack_.attn_decode_split = keys;
     }
   }
-  if (!c.first_stage || !c.final_stage) boundary_dev_.allocate(R * H_ * 2, "boundary");
   pin_items_.allocate(tokens_offset() + R * sizeof(int32_t));
   pin_out_tokens_.allocate((items_max_ + 1) * sizeof(int32_t));
   pin_sample_params_.allocate(items_max_ * sizeof(SampleParams));
@@ -1273,10 +1272,8 @@ void Stage::submit(const hllm_rocm_pass& pass, bool phases) {
                      embedding_.cols_padded, pack_.row_token, R, (int)H_, h);
       });
     } else {
-      HIP_CHECK(hipMemcpyAsync(boundary_dev_.ptr, pin_boundary_.ptr, (size_t)R * H_ * 2, hipMemcpyHostToDevice,
-                               stream_));
       timed("boundary", (uint64_t)R * H_ * 6, 0.0,
-            [&] { launch_boundary_decode(stream_, boundary_dev_.as<uint16_t>(), R, (int)H_, h); });
+            [&] { launch_boundary_decode(stream_, pin_boundary_.as<uint16_t>(), R, (int)H_, h); });
     }
     mark_phase(c_.first_stage ? "embedding" : "from-wire", -1);
     uint16_t* a0h = a0_hi_.as<uint16_t>();
@@ -1441,18 +1438,15 @@ void Stage::submit(const hllm_rocm_pass& pass, bool phases) {
       }
     } else {
       timed("boundary", (uint64_t)R * H_ * 6, 0.0, [&] {
-        launch_boundary_encode(stream_, h, R, (int)H_, pending, boundary_dev_.as<uint16_t>(), flags_dev());
+        launch_boundary_encode(stream_, h, R, (int)H_, pending, pin_boundary_.as<uint16_t>(), pin_flags());
       });
-      HIP_CHECK(hipMemcpyAsync(pin_boundary_.ptr, boundary_dev_.ptr, (size_t)R * H_ * 2, hipMemcpyDeviceToHost,
-                               stream_));
       mark_phase("to-wire", -1);
     }
-    // The sampled tokens (final stage) and the error flags behind them: one copy.
+    // The sampled tokens (final stage) and the error flags behind them: one copy. A boundary
+    // stage's flag is written with its rows; a final stage without sampled rows sets none.
     if (c_.final_stage && S > 0)
       HIP_CHECK(hipMemcpyAsync(pin_out_tokens_.ptr, tokens_.ptr, (items_max_ + 1) * sizeof(int32_t),
                                hipMemcpyDeviceToHost, stream_));
-    else
-      HIP_CHECK(hipMemcpyAsync(pin_flags(), flags_dev(), sizeof(int32_t), hipMemcpyDeviceToHost, stream_));
     HIP_CHECK(hipGetLastError());
   };
   // ---- the sequences' state, checked and claimed for this pass under one lock
@@ -1472,6 +1466,7 @@ void Stage::submit(const hllm_rocm_pass& pass, bool phases) {
     }
     for (uint32_t s : seqs) sequences_[s].in_flight = true;
   }
+  *pin_flags() = 0;
   phases_on_ = phases;
   for (const PhaseMark& m : phase_marks_) event_pool_.push_back(m.end);
   phase_marks_.clear();
