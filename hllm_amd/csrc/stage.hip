@@ -1,6 +1,9 @@
 // The stage runtime behind the C ABI: weights resident in HBM in the F-layout, a paged KV
 // pool with a host-side block allocator, per-pass workspaces reserved up front, and the
 // pass pipeline (pack -> embed/decode -> layers -> head/argmax or boundary encode).
+#include <sys/mman.h>
+#include <unistd.h>
+
 #include <algorithm>
 #include <cctype>
 #include <atomic>
@@ -24,6 +27,35 @@ namespace {
 thread_local std::string g_last_error;
 
 uint64_t pad_to(uint64_t x, uint64_t m) { return (x + m - 1) / m * m; }
+
+// Copies `count` F16 values and says whether all of them are finite. The test has no early exit,
+// so that it compiles to vector compares (an exit per element kept it scalar), and takes the
+// copy's blocks while they are in cache.
+bool copy_finite_halves(const uint16_t* in, uint64_t count, uint16_t* out) {
+  constexpr uint64_t kBlock = 8192;
+  for (uint64_t at = 0; at < count; at += kBlock) {
+    const uint64_t n = std::min(kBlock, count - at);
+    std::memcpy(out + at, in + at, n * sizeof(uint16_t));
+    uint16_t bad = 0;
+    for (uint64_t i = 0; i < n; ++i) bad |= (uint16_t)((in[at + i] & 0x7c00u) == 0x7c00u);
+    if (bad) return false;
+  }
+  return true;
+}
+
+// Maps the pages of a caller's output buffer before it is written: done while the GPU works, it
+// takes the page faults of fresh memory out of the copy that follows the pass. The contents do
+// not change; where the kernel has no such request the copy faults them in as before.
+void populate_pages(void* data, uint64_t bytes) {
+#ifdef MADV_POPULATE_WRITE
+  const uint64_t page = (uint64_t)sysconf(_SC_PAGESIZE);
+  const uint64_t first = ((uint64_t)data + page - 1) / page * page, end = ((uint64_t)data + bytes) / page * page;
+  if (end > first) (void)madvise(reinterpret_cast<void*>(first), end - first, MADV_POPULATE_WRITE);
+#else
+  (void)data;
+  (void)bytes;
+#endif
+}
 
 // Decode passes fuse QK-norm, RoPE and the K/V append into attention unless
 // HLLM_ROCM_ROPE_FUSION=0 (the separate kernel, for comparisons).
@@ -1189,11 +1221,8 @@ void Stage::submit(const hllm_rocm_pass& pass, bool phases) {
     }
   }
   if (!c_.first_stage) {
-    const uint64_t count = rows * H_;
-    for (uint64_t i = 0; i < count; ++i) {
-      if ((pass.boundary_in[i] & 0x7c00u) == 0x7c00u) fail(HLLM_INVALID_REQUEST, "non-finite activation");
-    }
-    std::memcpy(pin_boundary_.ptr, pass.boundary_in, count * 2);
+    if (!copy_finite_halves(pass.boundary_in, rows * H_, pin_boundary_.as<uint16_t>()))
+      fail(HLLM_INVALID_REQUEST, "non-finite activation");
   }
   if (cancel_requested(pass)) fail(HLLM_CANCELLED, "request cancelled");
   // Algorithmic attention bytes of one layer: every item's keys and values read once,
@@ -1539,6 +1568,7 @@ void Stage::wait(hllm_rocm_phase_time* phases, uint32_t capacity, uint32_t* coun
   std::unique_lock<std::mutex> lock(pass_mutex_);
   if (!in_flight_) fail(HLLM_INVALID_REQUEST, "no pass in flight");
   in_flight_ = false;
+  if (!c_.final_stage && pending_.boundary_out) populate_pages(pending_.boundary_out, pending_rows_ * H_ * 2);
   const hipError_t e = hipStreamSynchronize(stream_);
   if (e != hipSuccess) {
     fail_pass(pending_sequences_);
@@ -1765,6 +1795,18 @@ double measure_mfma_rate(int32_t device, uint32_t shape) {
   return best;
 }
 
+namespace {
+// A part of one device allocation.
+struct Area {
+  size_t at = 0, bytes = 0;
+  void* ptr = nullptr;
+  template <typename T>
+  T* as() const {
+    return static_cast<T*>(ptr);
+  }
+};
+}  // namespace
+
 void sample_logits(int32_t device, const float* logits, uint64_t rows, uint64_t V, const hllm_rocm_item* options,
                    uint64_t* tokens, double* logprobs, uint64_t* top_ids, double* top_logprobs) {
   if (!logits || !options || !tokens || rows == 0 || V == 0) fail(HLLM_INVALID_REQUEST, "invalid sampling request");
@@ -1786,27 +1828,33 @@ void sample_logits(int32_t device, const float* logits, uint64_t rows, uint64_t 
   } st;
   HIP_CHECK(hipStreamCreate(&st.s));
   const int blocks = (int)std::min<uint64_t>(rows, kSampleBlocks);
-  DeviceMemory d_logits, d_rows, d_tokens, d_flags, d_val, d_idx, d_params, d_out, d_w, d_lists, d_buckets, d_hist,
-      d_lse, d_sorted, d_cursor, d_candidates;
   int cus = 256;
   HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
   const int chunks = std::max(1, std::min(32, 4 * cus / blocks));
-  d_logits.allocate(rows * V * sizeof(float), "logits");
-  d_rows.allocate(sizeof(int32_t), "sampling");
-  d_tokens.allocate(rows * sizeof(int32_t), "sampling");
-  d_flags.allocate(sizeof(int32_t), "sampling");
-  d_val.allocate(rows * kArgmaxParts * sizeof(float), "argmax");
-  d_idx.allocate(rows * kArgmaxParts * sizeof(int32_t), "argmax");
-  d_params.allocate(rows * sizeof(SampleParams), "sampling");
-  d_out.allocate(rows * (6 * sizeof(double) + 5 * sizeof(int32_t)), "sampling");
-  d_w.allocate((size_t)blocks * V * sizeof(double), "sampling workspace");
-  d_lists.allocate((size_t)blocks * 4 * V * sizeof(uint32_t), "sampling workspace");
-  d_buckets.allocate((size_t)blocks * sample_bucket_stride(V), "sampling workspace");
-  d_hist.allocate((size_t)blocks * 256 * 3 * sizeof(uint64_t), "sampling workspace");
-  d_lse.allocate((size_t)blocks * chunks * sizeof(double), "sampling workspace");
-  d_sorted.allocate((size_t)blocks * V * sizeof(uint32_t), "sampling workspace");
-  d_cursor.allocate((size_t)blocks * 256 * sizeof(uint32_t), "sampling workspace");
-  d_candidates.allocate((size_t)blocks * chunks * 8 * sizeof(uint32_t), "sampling workspace");
+  // One allocation for the call's areas (one each, sixteen allocations and frees,
+  // took most of the call), 256-byte aligned.
+  size_t total = 0;
+  const auto area = [&](size_t bytes) {
+    Area a;
+    a.at = total;
+    a.bytes = bytes;
+    total += (bytes + 255) / 256 * 256;
+    return a;
+  };
+  Area d_logits = area(rows * V * sizeof(float)), d_rows = area(sizeof(int32_t)), d_tokens = area(rows * sizeof(int32_t)),
+       d_flags = area(sizeof(int32_t)), d_val = area(rows * kArgmaxParts * sizeof(float)),
+       d_idx = area(rows * kArgmaxParts * sizeof(int32_t)), d_params = area(rows * sizeof(SampleParams)),
+       d_out = area(rows * (6 * sizeof(double) + 5 * sizeof(int32_t))), d_w = area((size_t)blocks * V * sizeof(double)),
+       d_lists = area((size_t)blocks * 4 * V * sizeof(uint32_t)),
+       d_buckets = area((size_t)blocks * sample_bucket_stride(V)), d_hist = area((size_t)blocks * 256 * 3 * sizeof(uint64_t)),
+       d_lse = area((size_t)blocks * chunks * sizeof(double)), d_sorted = area((size_t)blocks * V * sizeof(uint32_t)),
+       d_cursor = area((size_t)blocks * 256 * sizeof(uint32_t)),
+       d_candidates = area((size_t)blocks * chunks * 8 * sizeof(uint32_t));
+  DeviceMemory memory;
+  memory.allocate(total, "sampling");
+  for (Area* a : {&d_logits, &d_rows, &d_tokens, &d_flags, &d_val, &d_idx, &d_params, &d_out, &d_w, &d_lists, &d_buckets,
+                  &d_hist, &d_lse, &d_sorted, &d_cursor, &d_candidates})
+    a->ptr = static_cast<unsigned char*>(memory.ptr) + a->at;
   HIP_CHECK(hipMemsetAsync(d_hist.ptr, 0, d_hist.bytes, st.s));
   HIP_CHECK(hipMemsetAsync(d_cursor.ptr, 0, d_cursor.bytes, st.s));
   const int32_t count = (int32_t)rows;
