@@ -1505,7 +1505,7 @@ Choice tile_choice(int rows, int n, uint64_t kp, bool deferred, size_t workspace
 //  - up to 64 rows: the register-streaming kernels (BM 16/32/64), except for very wide outputs
 //    (gate+up, LM head) with more than 32 rows, where staging the activations in LDS once per
 //    256-feature tile wins;
-//  - F16 passes from 224 rows: tile_choice;
+//  - F16 passes from 224 rows: tile_choice; F32 execution by the size of the weights;
 //  - the rest: the activation-staged kernel, BM 64, or BM 128 from 384 rows.
 // K is split while there are few output tiles. When the consumer sums the partials
 // (`deferred`) a split costs one partial write, so about 220-280 workgroups are targeted;
@@ -1536,10 +1536,25 @@ Choice gemm_choice(int rows, int n, uint64_t kp, bool deferred, bool f16, size_t
     const int config = rows <= 16 ? 0 : rows <= 32 ? 1 : 2;
     const int tiles = (n + 63) / 64;
     const int cap = std::max(1, (int)(kp >> 5) / 8);  // at least two k-steps per K-wave
-    return {config, deferred ? std::min(rounded(220.0 / tiles), cap) : 0};
+    // Unsplit where a quarter of the CUs have a tile: the reduce kernel behind a split costs
+    // more (F32 execution, gate+up of Qwen3-0.6B at 24 rows 15.9 -> 10.0 us).
+    return {config, deferred ? std::min(rounded(220.0 / tiles), cap) : tiles >= cus / 4 ? 1 : 0};
   }
-  // Wide outputs of 193-223 rows (and up to 768 in F32 execution): 128-row tiles, unsplit.
-  if (wide && !deferred && rows > 192 && rows <= 768) return {15, 1};
+  if (!f16) {
+    // F32 execution (split activations, two or three products per weight fragment): 16-row
+    // register-streaming tiles while their repeated weight reads stay small (the weights once
+    // per 16 rows, from L2), the activation-staged kernel's 32-row tiles from 224 to 1024 rows
+    // (128-row tiles win at 2048: 1177 / 1031 us per Qwen3-4B layer). Qwen3-0.6B
+    // at 96 rows against 64-row tiles: q/k/v 16.6 -> 10.6, o 15.2 -> 8.5, gate+up 24.4 -> 14.6, down
+    // 16.0 -> 9.2 us; at 120 MB the two meet (q/k/v 16.0 / 16.4 us at 224 rows; 157 MB of Qwen3-4B's
+    // at 65 rows 21.3 / 18.3). 32-row tiles, Qwen3-4B at 512 rows: 67 -> 47, 53 -> 38, 160 -> 119, 96 -> 74
+    // us per projection, at 224 rows 44 -> 30, 37 -> 24, 81 -> 73, 58 -> 44.
+    const double tile_reads = (rows + 15) / 16 * 2.0 * n * (double)kp;
+    if (tile_reads <= 120e6) return {0, 0};
+    if (rows >= 224 && rows <= 1024) return {11, deferred ? 0 : 1};
+  }
+  // Wide outputs of 193-223 rows: 128-row tiles, unsplit.
+  if (f16 && wide && !deferred && rows > 192) return {15, 1};
   const int bm = rows >= 384 || (wide && rows > 192) ? 128 : 64;
   const int config = bm == 128 ? 9 : 12;
   const int kc = bm == 128 ? 4 : 8;
