@@ -1600,12 +1600,17 @@ const DecodeShape& decode_shape(bool pair) {
   return pair ? paired : deferred;
 }
 
-// Whether the decode kernel runs this projection: F16, at most 64 rows, and either a consumer
-// that sums K splits, SwiGLU (never split), or enough output features to fill the GPU unsplit.
+// Whether the decode kernel runs this projection: F16, and at most 64 rows where a consumer
+// sums K splits or for SwiGLU (never split), or at most 128 rows with enough output features to
+// fill the GPU unsplit (the LM head: Qwen3-4B's at 128 rows 199 -> 172 us
+// against the activation-staged kernel, 4.5 TB/s).
 bool decode_applies(const GemmArgs& a, int prec, int rows, int cus) {
-  if (prec != kF16 || rows > 64 || rows <= 0) return false;
-  if (a.defer_reduce || a.epilogue == kEpiSwiglu) return true;
-  const int waves = decode_shape(false).waves >= 8 ? 8 : 4;
+  const bool summed = a.defer_reduce || a.epilogue == kEpiSwiglu;
+  if (prec != kF16 || rows > (summed ? 64 : 128) || rows <= 0) return false;
+  if (summed) return true;
+  const DecodeShape& d = decode_shape(false);
+  const int waves = d.waves >= 8 ? 8 : 4;
+  if (rows > 64 && (waves != 8 || d.frags != 1)) return false;  // its only shape above 64 rows
   const int n_tiles = (a.N + 16 * waves - 1) / (16 * waves);
   return n_tiles * waves >= 4 * cus;
 }
@@ -1692,7 +1697,8 @@ int launch_decode(hipStream_t stream, const GemmArgs& a, int rows, int cus) {
   }
   if (rows <= 16) return launch_decode_rows<1>(stream, a, cus);
   if (rows <= 32) return launch_decode_rows<2>(stream, a, cus);
-  return launch_decode_rows<4>(stream, a, cus);
+  if (rows <= 64) return launch_decode_rows<4>(stream, a, cus);
+  return launch_decode_waves<8, 1, 4, 4, false, 4>(stream, a, 8, 1);  // unsplit outputs (decode_applies)
 }
 
 std::atomic<int>& forced_config() {
