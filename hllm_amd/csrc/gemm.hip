@@ -1236,6 +1236,132 @@ __global__ void __launch_bounds__(64 * WAVES) gemm_decode_kernel(GemmArgs a, int
   }
 }
 
+// The operand's RMSNorm computed by every workgroup of the projection (GemmArgs::norm), row by
+// row, with Q chunks of four columns per thread: a launch of its own is a chain of two memory
+// round trips and a kernel boundary, 4 us per norm of one row, and here the weights' first loads
+// (`prefetch`) are in flight behind it. Every workgroup reads the rows and their partials, so it
+// pays for one or two rows only. put(row, column, four halves) stores the operand.
+template <int NT, int Q, typename Prefetch, typename Put>
+__device__ inline void fold_norm_row(const NormFold& f, int row, bool publish, float* scratch, Prefetch&& prefetch,
+                                     Put&& put) {
+  constexpr int U = 12 / Q;  // partials' loads in flight at once, at clamped addresses
+  const int wave = threadIdx.x >> 6;
+  floatx4 v[Q], w[Q], y[Q];
+  int c[Q], at[Q];
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    c[q] = 4 * ((int)threadIdx.x + q * NT);
+    at[q] = min(c[q], f.hidden - 4);
+    v[q] = *reinterpret_cast<const floatx4*>(f.h + (size_t)row * f.hidden + at[q]);
+    w[q] = *reinterpret_cast<const floatx4*>(f.weight + at[q]);
+    y[q] = floatx4{0.f, 0.f, 0.f, 0.f};
+  }
+  const float* base = (f.parts > 0 ? f.partials : f.h) + (size_t)row * f.hidden;
+  floatx4 p[U][Q];
+  int s0 = 0;
+  const auto load = [&] {
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int q = 0; q < Q; ++q)
+        p[u][q] = *reinterpret_cast<const floatx4*>(base + (size_t)max(0, min(s0 + u, f.parts - 1)) * f.stride + at[q]);
+  };
+  const auto sum = [&] {
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int q = 0; q < Q; ++q)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) y[q][j] = s0 + u < f.parts ? y[q][j] + p[u][q][j] : y[q][j];
+  };
+  load();
+  while (s0 + U < f.parts) {
+    sum();
+    s0 += U;
+    load();
+  }
+  prefetch();
+  sum();
+  float squares = 0.0f;
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    const bool in = c[q] < f.hidden;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      v[q][j] += y[q][j];
+      squares += in ? v[q][j] * v[q][j] : 0.0f;
+    }
+    if (publish && f.h_out && in) *reinterpret_cast<floatx4*>(f.h_out + (size_t)row * f.hidden + c[q]) = v[q];
+  }
+  for (int o = 32; o > 0; o >>= 1) squares += __shfl_xor(squares, o, 64);
+  if ((threadIdx.x & 63) == 0) scratch[wave] = squares;
+  __syncthreads();
+  float total = 0.0f;
+#pragma unroll
+  for (int t = 0; t < NT / 64; ++t) total += scratch[t];
+  __syncthreads();
+  const float inverse = 1.0f / sqrtf(total / (float)f.hidden + f.eps);
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    if (c[q] >= f.hidden) continue;
+    half4 x;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) x[j] = to_half((v[q][j] * inverse) * w[q][j]);
+    put(row, c[q], x);
+  }
+}
+
+// gemm_decode_kernel's deferred projection (eight waves of one fragment row, the split's
+// operand whole in LDS) for the one or two rows of a folded RMSNorm.
+template <int Q>
+__global__ void __launch_bounds__(512) gemm_norm_kernel(GemmArgs a, int n_tiles) {
+  constexpr int P = 4;
+  extern __shared__ float lds[];  // the split's fragments [per][64] half8, then 8 floats
+  half8* xs = reinterpret_cast<half8*>(lds);
+  const int tile_n = blockIdx.x % n_tiles, split = blockIdx.x / n_tiles;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int KT = (int)(a.Kp >> 5);
+  const int per = ((KT + a.ksplit - 1) / a.ksplit + P - 1) / P * P;
+  const int kt0 = split * per, kt1 = min(KT, kt0 + per);
+  const int steps = kt1 > kt0 ? kt1 - kt0 : 0, kt_last = max(0, kt1 - 1);
+  const int frag = tile_n * 8 + wave;
+  const half8* W = reinterpret_cast<const half8*>(a.w_hi) + (size_t)frag * KT * 64 + lane;
+  half8 rw[P];
+  const auto load_w = [&](int slot, int kt) { rw[slot] = __builtin_nontemporal_load(W + (size_t)min(kt, kt_last) * 64); };
+  const auto put = [&](int row, int c, half4 x) {
+    const int s = (c >> 5) - kt0;
+    if (s >= 0 && s < steps)
+      *reinterpret_cast<half4*>(reinterpret_cast<_Float16*>(xs + s * 64 + row + ((c & 31) >> 3) * 16) + (c & 7)) = x;
+  };
+  float* scratch = lds + (size_t)per * 256;
+  fold_norm_row<512, Q>(
+      a.norm, 0, blockIdx.x == 0, scratch,
+      [&] {
+#pragma unroll
+        for (int s = 0; s < P; ++s) load_w(s, kt0 + s);
+      },
+      put);
+  for (int row = 1; row < a.M; ++row) fold_norm_row<512, Q>(a.norm, row, blockIdx.x == 0, scratch, [] {}, put);
+  __syncthreads();
+  // Lanes of rows past M read LDS that nothing wrote: their columns are never stored.
+  floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < steps; s0 += P) {
+#pragma unroll
+    for (int j = 0; j < P; ++j) {
+      if (s0 + j < steps) acc = mfma(rw[j], xs[(s0 + j) * 64 + lane], acc);
+      load_w(j, kt0 + s0 + j + P);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  const int row = lane & 15, col = frag * 16 + (lane >> 4) * 4;
+  if (row >= a.M || col >= a.N) return;
+  const bool partial = a.ksplit > 1;
+  float* dst = partial ? a.workspace + ((size_t)split * a.M + row) * a.N + col : a.out + (size_t)row * a.ldo + col;
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+    if (col + t < a.N) dst[t] = acc[t];
+}
+
 // Gate/up projection of few rows (F16, SwiGLU), HBM- and latency-bound: a workgroup owns NP
 // gate/up pairs of 16 features and its WK waves interleave the k-steps, each streaming its own
 // weight and activation fragments through a ring of P k-steps; the waves' tiles are summed
@@ -1244,10 +1370,11 @@ __global__ void __launch_bounds__(64 * WAVES) gemm_decode_kernel(GemmArgs a, int
 // activations once per workgroup. Qwen3-0.6B, 12.6 MB of weights: 8.75 -> 5.1 us for one row
 // (1.4 -> 2.5 TB/s), 11.1 -> 6.1 us for 45; 67 MB at K 2 048, seven rows: 17.9 -> 13.9 us
 // (4.8 TB/s). WK 8 and rings of 8 measured the same or up to 1.5 us slower.
-template <int MF, int NP, int WK, int P>
+// Q > 0: the operand is the folded RMSNorm of one or two rows (fold_norm_row), row-major in LDS.
+template <int MF, int NP, int WK, int P, int Q>
 __global__ void __launch_bounds__(64 * WK) gemm_pair_kernel(GemmArgs a) {
   constexpr int NF = 2 * NP;
-  extern __shared__ float lds[];  // [WK][MF][NF][64] floatx4
+  extern __shared__ float lds[];  // [WK][MF][NF][64] floatx4, then (Q > 0) [kFoldRows][Kp] halves and WK floats
   const int M = a.device_m ? *a.device_m : a.M;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int KT = (int)(a.Kp >> 5);
@@ -1271,31 +1398,49 @@ __global__ void __launch_bounds__(64 * WK) gemm_pair_kernel(GemmArgs a) {
   // Unconditional loads (see gemm_kernel); past the range they re-read the last k-step.
   auto load = [&](int slot, int step) {
     const int kt = min(wave + step * WK, KT - 1);
+    if constexpr (Q == 0) {
 #pragma unroll
-    for (int i = 0; i < MF; ++i) rx[slot][i] = X[i * frag_stride + (size_t)kt * 64];
+      for (int i = 0; i < MF; ++i) rx[slot][i] = X[i * frag_stride + (size_t)kt * 64];
+    }
 #pragma unroll
     for (int j = 0; j < NF; ++j) rb[slot][j] = __builtin_nontemporal_load(W[j] + (size_t)kt * 64);
   };
-  auto compute = [&](int s) {
+  _Float16* xs = reinterpret_cast<_Float16*>(lds + (size_t)WK * MF * NF * 256);
+  // Lanes of rows past M repeat the last one: their columns are never stored.
+  const _Float16* xrow = xs + (size_t)min(lane & 15, M - 1) * a.Kp + (lane >> 4) * 8;
+  auto compute = [&](int s, int step) {
+    if constexpr (Q > 0) rx[s][0] = *reinterpret_cast<const half8*>(xrow + (wave + step * WK) * 32);
 #pragma unroll
     for (int i = 0; i < MF; ++i)
 #pragma unroll
       for (int j = 0; j < NF; ++j) acc[i][j] = mfma(rb[s][j], rx[s][i], acc[i][j]);
   };
+  const auto fill = [&] {
 #pragma unroll
-  for (int s = 0; s < P; ++s) load(s, s);
+    for (int s = 0; s < P; ++s) load(s, s);
+  };
+  if constexpr (Q > 0) {
+    static_assert(MF == 1, "folded rows are one row tile");
+    float* scratch = reinterpret_cast<float*>(xs + (size_t)kFoldRows * a.Kp);
+    const auto put = [&](int row, int c, half4 x) { *reinterpret_cast<half4*>(xs + (size_t)row * a.Kp + c) = x; };
+    fold_norm_row<64 * WK, Q>(a.norm, 0, blockIdx.x == 0, scratch, fill, put);
+    for (int row = 1; row < M; ++row) fold_norm_row<64 * WK, Q>(a.norm, row, blockIdx.x == 0, scratch, [] {}, put);
+    __syncthreads();
+  } else {
+    fill();
+  }
   int base = 0;
   for (; base + P < steps; base += P) {
 #pragma unroll
     for (int s = 0; s < P; ++s) {
-      compute(s);
+      compute(s, base + s);
       load(s, base + s + P);
       __builtin_amdgcn_sched_barrier(0);
     }
   }
 #pragma unroll
   for (int s = 0; s < P; ++s)
-    if (base + s < steps) compute(s);
+    if (base + s < steps) compute(s, base + s);
 
   floatx4* tiles = reinterpret_cast<floatx4*>(lds);
 #pragma unroll
@@ -1326,19 +1471,21 @@ __global__ void __launch_bounds__(64 * WK) gemm_pair_kernel(GemmArgs a) {
   }
 }
 
-template <int MF, int NP, int WK, int P>
+template <int MF, int NP, int WK, int P, int Q = 0>
 void launch_pair_shape(hipStream_t stream, const GemmArgs& a) {
   if ((uint64_t)MF * 16 > a.x_rows_padded) fail(HLLM_INTERNAL, "GEMM tile exceeds the activation padding");
   if (a.N % (32 * NP) != 0 || (uint64_t)a.N > a.w_rows_padded) fail(HLLM_INTERNAL, "gate/up pairs exceed the weights");
-  constexpr size_t lds = (size_t)WK * MF * NP * 2 * 1024;
+  constexpr size_t tiles = (size_t)WK * MF * NP * 2 * 1024;
+  constexpr size_t most = tiles + (Q > 0 ? kFoldRows * kFoldHidden * 2 + WK * 4 : 0);
   static const bool configured = [] {
-    HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_pair_kernel<MF, NP, WK, P>),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_pair_kernel<MF, NP, WK, P, Q>),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)most));
     return true;
   }();
   (void)configured;
-  observed(kernel_name<MF, NP, WK, P>("gemm_pair_kernel"),
-           [&] { gemm_pair_kernel<MF, NP, WK, P><<<dim3(a.N / (32 * NP)), 64 * WK, lds, stream>>>(a); });
+  const size_t lds = tiles + (Q > 0 ? kFoldRows * a.Kp * 2 + WK * 4 : 0);
+  observed(kernel_name<MF, NP, WK, P, Q>("gemm_pair_kernel"),
+           [&] { gemm_pair_kernel<MF, NP, WK, P, Q><<<dim3(a.N / (32 * NP)), 64 * WK, lds, stream>>>(a); });
 }
 
 // LDS a decode workgroup may give to its split's whole activation range.
@@ -1635,6 +1782,15 @@ int decode_frags(const GemmArgs& a, int waves) {
   return nfw;
 }
 
+// K splits of a deferred decode projection over `chunks` chunks of k-steps and n_tiles
+// workgroups of `waves` waves: splits of whole chunks, none of them empty.
+int decode_splits(int chunks, int n_tiles, int waves, int cus) {
+  const double want = (double)decode_shape(false).target_waves_per_cu * cus / ((double)n_tiles * waves);
+  const int ksplit = std::max(1, std::min((int)(want + 0.5), chunks / 2 > 0 ? chunks / 2 : 1));
+  const int per = (chunks + ksplit - 1) / ksplit;
+  return (chunks + per - 1) / per;
+}
+
 template <int MF, int KC, int P, int PW>
 int launch_decode_variant(hipStream_t stream, const GemmArgs& a, int cus) {
   const bool pair = a.epilogue == kEpiSwiglu;
@@ -1645,13 +1801,7 @@ int launch_decode_variant(hipStream_t stream, const GemmArgs& a, int cus) {
   const int fr = waves * nfw;
   const int n_tiles = (a.N + 16 * fr - 1) / (16 * fr);
   int ksplit = 1;
-  if (a.defer_reduce) {
-    // Splits of whole chunks, none of them empty.
-    const double want = (double)d.target_waves_per_cu * cus / ((double)n_tiles * waves);
-    ksplit = std::max(1, std::min((int)(want + 0.5), chunks / 2 > 0 ? chunks / 2 : 1));
-    const int per = (chunks + ksplit - 1) / ksplit;
-    ksplit = (chunks + per - 1) / per;
-  }
+  if (a.defer_reduce) ksplit = decode_splits(chunks, n_tiles, waves, cus);
   if constexpr (MF > 1) {  // one row tile: the pair kernel
     if (pair) return launch_decode_waves<MF, 2, KC, P, true, P>(stream, a, waves, 1);
   }
@@ -1681,6 +1831,39 @@ void launch_pair(hipStream_t stream, const GemmArgs& a, int cus) {
     if (a.N / 32 > cus) return launch_pair_shape<MF, 2, 4, 4>(stream, a);
   }
   launch_pair_shape<MF, 1, 4, 4>(stream, a);
+}
+
+// A projection with its operand's RMSNorm folded in (gemm_folds_norm): returns the partials left.
+int launch_folded(hipStream_t stream, GemmArgs a, int cus) {
+  if (a.epilogue == kEpiSwiglu) {
+    switch ((a.norm.hidden + 1023) / 1024) {
+      case 1: launch_pair_shape<1, 1, 4, 4, 1>(stream, a); break;
+      case 2: launch_pair_shape<1, 1, 4, 4, 2>(stream, a); break;
+      case 3: launch_pair_shape<1, 1, 4, 4, 3>(stream, a); break;
+      default: launch_pair_shape<1, 1, 4, 4, 4>(stream, a); break;
+    }
+    return 0;
+  }
+  const int n_tiles = (a.N + 127) / 128, KT = (int)(a.Kp >> 5), chunks = (KT + 3) / 4;
+  if ((uint64_t)n_tiles * 128 > a.w_rows_padded) fail(HLLM_INTERNAL, "GEMM tile exceeds the weight padding");
+  a.ksplit = decode_splits(chunks, n_tiles, 8, cus);
+  if ((size_t)a.ksplit * a.M * a.N > a.workspace_floats) a.ksplit = 1;
+  const int per = ((KT + a.ksplit - 1) / a.ksplit + 3) / 4 * 4;
+  const size_t lds = (size_t)per * 1024 + 8 * sizeof(float);
+  const auto go = [&](auto kernel, const char* name) {
+    static const bool configured = [kernel] {
+      HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    160 * 1024));
+      return true;
+    }();
+    (void)configured;
+    observed(name, [&] { kernel<<<dim3(n_tiles * a.ksplit), 512, lds, stream>>>(a, n_tiles); });
+  };
+  if (a.norm.hidden <= 2048)
+    go(&gemm_norm_kernel<1>, "gemm_norm_kernel<1>");
+  else
+    go(&gemm_norm_kernel<2>, "gemm_norm_kernel<2>");
+  return a.ksplit > 1 ? a.ksplit : 0;
 }
 
 int launch_decode(hipStream_t stream, const GemmArgs& a, int rows, int cus) {
@@ -1714,6 +1897,18 @@ int set_forced_gemm_config(int config) { return forced_config().exchange(config)
 
 int forced_gemm_config() { return forced_config().load(std::memory_order_relaxed); }
 
+// (HLLM_ROCM_NORM_FOLD=0, read at every call, says false, for comparisons.)
+bool gemm_folds_norm(const GemmArgs& a, int prec, int rows, int hidden, int cus) {
+  // Every workgroup normalises the rows one after the other: at 2 rows of 2560 and 3072 columns the
+  // passes took 0-2% longer than with separate norms (one row of them 6-7% less; Qwen3-0.6B 573 -> 478
+  // us for one row on fourteen layers and 600 -> 537 for two, 2048 columns 650 -> 575 and 655 -> 627).
+  if (rows > kFoldRows || rows * hidden > kFoldHidden || (uint64_t)hidden != a.Kp) return false;
+  if (forced_config().load(std::memory_order_relaxed) >= 0 || env_int("HLLM_ROCM_DECODE_OFF", 0) != 0 ||
+      env_int("HLLM_ROCM_DECODE_WHOLE", 1) == 0 || env_int("HLLM_ROCM_NORM_FOLD", 1) == 0)
+    return false;
+  return decode_applies(a, prec, rows, cus) && (a.epilogue == kEpiSwiglu ? pair_applies(a, rows, cus) : a.epilogue == kEpiStore && a.defer_reduce != 0);
+}
+
 int gemm_argmax_parts(const GemmArgs& a, int prec, int rows_bound, int cus) {
   if (env_int("HLLM_ROCM_FUSED_ARGMAX", 1) == 0 || a.defer_reduce || a.epilogue == kEpiSwiglu) return 0;
   const int forced = forced_config().load(std::memory_order_relaxed);
@@ -1726,6 +1921,10 @@ int gemm_argmax_parts(const GemmArgs& a, int prec, int rows_bound, int cus) {
 int launch_gemm(hipStream_t stream, const GemmArgs& args, int prec, int rows_bound, int cus) {
   if (rows_bound <= 0) return 0;
   const int forced = forced_config().load(std::memory_order_relaxed);
+  if (args.norm.h) {
+    if (!gemm_folds_norm(args, prec, rows_bound, args.norm.hidden, cus)) fail(HLLM_INTERNAL, "the projection cannot fold its norm");
+    return launch_folded(stream, args, cus);
+  }
   if (args.epilogue == kEpiArgmax) {
     // Only the decode kernel has the argmax epilogue (gemm_argmax_parts says when it runs).
     if (gemm_argmax_parts(args, prec, rows_bound, cus) != args.argmax_parts || args.argmax_parts <= 0)

@@ -13,6 +13,21 @@ enum Epilogue : int {
                      // (argmax_val / argmax_idx [m][parts], parts = gemm_argmax_parts)
 };
 
+// The RMSNorm that makes a projection's operand, folded into the projection (few rows of F16
+// execution, gemm_folds_norm): row r is h[r] plus the partials in split order, normalised and
+// scaled by `weight`; the sums are written to h_out (not h: other workgroups read it) when set.
+struct NormFold {
+  const float* h = nullptr;  // nullptr: x_hi holds the operand
+  float* h_out = nullptr;
+  const float* weight = nullptr;
+  const float* partials = nullptr;
+  int parts = 0;
+  uint64_t stride = 0;
+  int hidden = 0;
+  float eps = 0.0f;
+};
+constexpr int kFoldRows = 2, kFoldHidden = 4096;  // at most 2 rows and 4096 columns in all
+
 struct GemmArgs {
   const uint16_t* w_hi;        // F-layout weights [N rows][Kp]
   const uint16_t* w_lo;        // lo parts (F32 residency) or nullptr
@@ -40,6 +55,7 @@ struct GemmArgs {
   int32_t* argmax_idx;
   int32_t* argmax_flags;       // bit 1 set when an output is not finite
   int argmax_parts;
+  NormFold norm;
 };
 
 // Activation rows a buffer needs so that every row tile of a launch over up to `rows`
@@ -48,6 +64,8 @@ inline uint64_t gemm_padded_rows(uint64_t rows) { return (rows + 256 + 127) / 12
 // Returns 0 when the epilogue has been applied, or (defer_reduce only) the number of K-split
 // partial output matrices left in the workspace for the consumer to sum in order.
 int launch_gemm(hipStream_t stream, const GemmArgs& args, int prec, int rows_bound, int cus);
+// Whether launch_gemm takes the operand's RMSNorm (GemmArgs::norm) for this projection.
+bool gemm_folds_norm(const GemmArgs& args, int prec, int rows, int hidden, int cus);
 // An explicit configuration of the table in gemm.hip (tuning), optionally forcing the K split.
 int launch_gemm_config(hipStream_t stream, const GemmArgs& args, int prec, int rows_bound, int cus,
                         int config, int forced_ksplit);

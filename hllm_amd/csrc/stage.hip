@@ -257,7 +257,7 @@ class Stage {
   int gemm(const char* family, const Matrix& w, const uint16_t* x_hi, const uint16_t* x_lo, int rows,
             int n, int epilogue, float* out, int ldo, uint16_t* out_hi, uint16_t* out_lo,
             uint64_t out_cols_padded,
-           bool defer = false, int argmax_parts = 0);
+            bool defer = false, int argmax_parts = 0, const NormFold& norm = {});
   template <typename F>
   void timed(const char* family, uint64_t bytes, double flops, F&& launch);
   hipEvent_t take_event();
@@ -485,7 +485,7 @@ Stage::Stage(const hllm_rocm_stage_config& c) : c_(c) {
 
   // ---- workspaces
   const size_t R = rows_padded_;
-  h_.allocate(R * H_ * sizeof(float), "hidden");
+  h_.allocate((R + kFoldRows) * H_ * sizeof(float), "hidden");  // the rows, then folded norms' spare rows
   const uint64_t a0_cols = Hp_, a1_cols = std::max(QDp_, Ip_);
   a0_hi_.allocate(R * a0_cols * 2, "operand");
   a1_hi_.allocate(R * a1_cols * 2, "operand");
@@ -1104,7 +1104,7 @@ std::string Stage::profile_records() {
 // consumer and their count is returned (0: the epilogue has been applied).
 int Stage::gemm(const char* family, const Matrix& w, const uint16_t* x_hi, const uint16_t* x_lo,
                 int rows, int n, int epilogue, float* out, int ldo, uint16_t* out_hi,
-                uint16_t* out_lo, uint64_t out_cols_padded, bool defer, int argmax_parts) {
+                uint16_t* out_lo, uint64_t out_cols_padded, bool defer, int argmax_parts, const NormFold& norm) {
   GemmArgs a{};
   a.defer_reduce = defer ? 1 : 0;
   a.w_hi = w.hi.as<uint16_t>();
@@ -1126,6 +1126,12 @@ int Stage::gemm(const char* family, const Matrix& w, const uint16_t* x_hi, const
   a.out_hi = out_hi;
   a.out_lo = out_lo;
   a.out_cols_padded = out_cols_padded;
+  a.norm = norm;
+  if (norm.h) {
+    // The norm reads the first half's partials while these are written.
+    a.workspace_floats = gemm_ws_floats_ / 2;
+    a.workspace += a.workspace_floats;
+  }
   if (argmax_parts > 0) {
     a.argmax_val = argmax_val_.as<float>();
     a.argmax_idx = argmax_idx_.as<int32_t>();
@@ -1286,6 +1292,21 @@ void Stage::submit(const hllm_rocm_pass& pass, bool phases) {
     fused_parts = gemm_argmax_parts(probe, prec_, S, cus_);
     if ((uint64_t)fused_parts * S > argmax_capacity_) fused_parts = 0;
   }
+  // Passes of one or two rows fold the layers' RMSNorms into q/k/v and gate+up.
+  bool fold_qkv = false, fold_gate_up = false;
+  if (R <= kFoldRows && L_ > 0) {
+    GemmArgs probe{};
+    probe.defer_reduce = 1;
+    probe.epilogue = kEpiStore;
+    probe.N = (int)qkv_n_;
+    probe.Kp = layers_[0]->qkv.cols_padded;
+    probe.w_rows_padded = layers_[0]->qkv.rows_padded;
+    fold_qkv = gemm_folds_norm(probe, prec_, R, (int)H_, cus_);
+    probe.defer_reduce = 0;
+    probe.epilogue = kEpiSwiglu;
+    probe.N = (int)(2 * Ip_);
+    fold_gate_up = gemm_folds_norm(probe, prec_, R, (int)H_, cus_);
+  }
   auto enqueue = [&](bool capturing) {
     // The item list (all slots) and, on the first stage, the pass's tokens: one copy.
     HIP_CHECK(hipMemcpyAsync(items_dev_.ptr, meta, tokens_offset() + (c_.first_stage ? R * sizeof(int32_t) : 0),
@@ -1316,30 +1337,39 @@ void Stage::submit(const hllm_rocm_pass& pass, bool phases) {
     // by RoPE/append, o's and down's (residual adds) by the next RMSNorm. `pending` holds
     // the previous layer's down-projection partials until this layer's input norm.
     float* ws = gemm_ws_.as<float>();
+    float* qkv_ws = fold_qkv ? ws + gemm_ws_floats_ / 2 : ws;
     Partials pending{};
+    // A folded norm: the rows it completes (those with partials) move to the spare rows.
+    float* spare = h + rows_padded_ * H_;
+    const auto fold_norm = [&](const DeviceMemory& weight, const Partials& p) {
+      return NormFold{h, p.parts > 0 ? spare : nullptr, weight.as<float>(), p.data, p.parts, p.stride, (int)H_, eps};
+    };
     for (uint64_t l = 0; l < L_; ++l) {
       if (!capturing && cancel_requested(pass)) fail(HLLM_CANCELLED, "request cancelled");
       Layer& w = *layers_[l];
-      timed("norm", (uint64_t)R * H_ * 6, 0.0, [&] {
-        launch_rmsnorm_flayout(stream_, h, (int)H_, nullptr, R, nullptr, w.input_norm.as<float>(), eps, a0h, a0l,
-                               Hp_, pending);
-      });
-      pending = {};
+      if (!fold_qkv)
+        timed("norm", (uint64_t)R * H_ * 6, 0.0, [&] {
+          launch_rmsnorm_flayout(stream_, h, (int)H_, nullptr, R, nullptr, w.input_norm.as<float>(), eps, a0h, a0l,
+                                 Hp_, pending);
+        });
       const int qkv_parts = gemm("gemm_qkv", w.qkv, a0h, a0l, R, (int)qkv_n_, kEpiStore, qkv_.as<float>(),
-                                 (int)qkv_n_, nullptr, nullptr, 0, true);
+                                 (int)qkv_n_, nullptr, nullptr, 0, true, 0,
+                                 fold_qkv ? fold_norm(w.input_norm, pending) : NormFold{});
+      if (fold_qkv && pending.parts > 0) std::swap(h, spare);
+      pending = {};
       if (!fuse_rope) {
         timed("rope_append", (uint64_t)R * qkv_n_ * 6, 0.0, [&] {
           launch_qkv_rope_append(stream_, qkv_.as<float>(), R, (int)Q_, (int)K_, (int)D_,
                                  c_.query_key_norm ? w.q_norm.as<float>() : nullptr,
                                  c_.query_key_norm ? w.k_norm.as<float>() : nullptr, eps, rope_cos_.as<float>(),
                                  rope_sin_.as<float>(), pack_.row_position, pack_.row_slot, kv_, (int)l,
-                                 q_.as<float>(), Partials{ws, qkv_parts, (uint64_t)R * qkv_n_});
+                                 q_.as<float>(), Partials{qkv_ws, qkv_parts, (uint64_t)R * qkv_n_});
         });
       }
       AttentionArgs at{};
       if (fuse_rope) {
         at.rope.qkv = qkv_.as<float>();
-        at.rope.parts = Partials{ws, qkv_parts, (uint64_t)R * qkv_n_};
+        at.rope.parts = Partials{qkv_ws, qkv_parts, (uint64_t)R * qkv_n_};
         at.rope.q_norm = c_.query_key_norm ? w.q_norm.as<float>() : nullptr;
         at.rope.k_norm = c_.query_key_norm ? w.k_norm.as<float>() : nullptr;
         at.rope.eps = eps;
@@ -1376,11 +1406,15 @@ void Stage::submit(const hllm_rocm_pass& pass, bool phases) {
       timed("attention", attn_bytes, attn_flops, [&] { launch_attention(stream_, at); });
       const int o_parts = gemm("gemm_o", w.o, a1h, a1l, R, (int)H_, kEpiResidual, h, (int)H_, nullptr, nullptr, 0,
                                true);
-      timed("norm", (uint64_t)R * H_ * 6, 0.0, [&] {
-        launch_rmsnorm_flayout(stream_, h, (int)H_, nullptr, R, nullptr, w.post_norm.as<float>(), eps, a0h, a0l,
-                               Hp_, Partials{ws, o_parts, (uint64_t)R * H_});
-      });
-      gemm("gemm_gate_up", w.gate_up, a0h, a0l, R, (int)(2 * Ip_), kEpiSwiglu, nullptr, 0, a1h, a1l, Ip_);
+      const Partials o_partials{ws, o_parts, (uint64_t)R * H_};
+      if (!fold_gate_up)
+        timed("norm", (uint64_t)R * H_ * 6, 0.0, [&] {
+          launch_rmsnorm_flayout(stream_, h, (int)H_, nullptr, R, nullptr, w.post_norm.as<float>(), eps, a0h, a0l,
+                                 Hp_, o_partials);
+        });
+      gemm("gemm_gate_up", w.gate_up, a0h, a0l, R, (int)(2 * Ip_), kEpiSwiglu, nullptr, 0, a1h, a1l, Ip_, false, 0,
+           fold_gate_up ? fold_norm(w.post_norm, o_partials) : NormFold{});
+      if (fold_gate_up && o_parts > 0) std::swap(h, spare);
       // The last layer's down partials are summed by the final norm, for the sampled rows it
       // gathers (nothing reads the other rows' residual afterwards), or by the boundary's
       // encoding.

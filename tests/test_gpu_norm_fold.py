@@ -1,0 +1,52 @@
+"""Passes of one and two rows, whose RMSNorms are folded into q/k/v and gate+up, against the oracle
+and beside passes of three rows (separate norms): row lengths around the chunk counts of both
+kernels, more partials than one round of loads, several layers (the residual rows alternate
+between two buffers), and both ends (final norm and head; boundary rows).
+
+Logits and boundary rows within max-abs 2e-2 and cosine 0.9999, as for the other F16 slices."""
+import numpy as np
+import pytest
+
+import oracle
+from hllm_amd import capi, model, synthetic
+from tests import helpers_parity as hp
+from tests import models
+
+pytestmark = pytest.mark.gpu
+PROMPT, STEPS, VOCAB = 5, 3, 300
+
+
+@pytest.mark.parametrize("hidden,intermediate,final", [
+    (64, 96, True), (1024, 160, False), (1056, 1600, True), (2048, 96, True), (2080, 352, False), (3104, 544, True),
+    (4096, 2080, False)])
+def test_folded_norms_match_the_oracle(hidden, intermediate, final):
+    shape = synthetic.ModelShape(f"h{hidden}", 3, hidden, intermediate, 4, 2, 64, VOCAB, eps=1e-6, theta=1e4,
+                                 qk_norm=False, tied=False, max_seq=64)
+    end = 3 if final else 2
+    st = capi.Stage(model.stage_config(shape, 0, end, first=True, final=final, execution="f16",
+                                       kv_cache_bytes=16 << 20, max_sequences=8, max_pass_rows=64))
+    model.synthesize(st, shape, seed=5, norm_sigma=0.1)
+    ost = oracle.OracleStage(models.synthetic_stage(shape, 0, end, first=True, final=final, seed=5, norm_sigma=0.1))
+    rng = np.random.default_rng(3)
+    for rows in (1, 2, 3):
+        ids = rng.integers(0, VOCAB, (PROMPT + STEPS, rows)).astype(np.uint64)
+        seqs = [st.allocate(PROMPT + STEPS) for _ in range(rows)]
+        oseqs = [ost.allocate_sequence(PROMPT + STEPS) for _ in range(rows)]
+        for r in range(rows):
+            st.execute([capi.item(seqs[r], PROMPT, 0, sample=False)], token_ids=ids[:PROMPT, r])
+            ost.execute(np.ascontiguousarray(ids[:PROMPT, r]), 0, oseqs[r])
+        for step in range(STEPS):
+            hp.say(shape.name, "rows", rows, "step", step)
+            position = PROMPT + step
+            out = st.execute([capi.item(s, 1, position, sample=final) for s in seqs], token_ids=ids[position],
+                             want_logits=final)
+            expect = []
+            for r in range(rows):
+                trace = []
+                result = ost.execute(ids[position, r:r + 1].copy(), position, oseqs[r], trace)
+                expect.append(trace[-1] if final else oracle.f16_decode(result[1])[0])
+            got = out["logits"] if final else oracle.f16_decode(out["boundary"])
+            hp.check_rows(got, np.stack(expect), (shape.name, rows, step))
+        for s in seqs:
+            st.release(s)
+    st.close()
