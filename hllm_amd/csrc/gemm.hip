@@ -523,8 +523,9 @@ __global__ void __launch_bounds__(256, PREC == kF16 && MF <= 8 ? 2 : 1)
   }
 }
 
-// Sum of a tile's K-split partials (in split order) plus the epilogue. One thread per 8
-// consecutive outputs of one row (8 activations for SwiGLU).
+// Sum of a tile's K-split partials (in split order), stored or through SwiGLU (residual
+// projections leave their partials to the next kernel). One thread per 8 consecutive outputs of
+// one row (8 activations for SwiGLU).
 template <int BM, int BN>
 __global__ void __launch_bounds__(256) gemm_reduce_kernel(GemmArgs a, int n_tiles, int tiles) {
   const int M = a.device_m ? *a.device_m : a.M;
@@ -608,12 +609,7 @@ __global__ void __launch_bounds__(256) gemm_reduce_kernel(GemmArgs a, int n_tile
   float* out = a.out + (size_t)gm * a.ldo + gn;
 #pragma unroll
   for (int t = 0; t < 8; ++t) {
-    if (gn + t < a.N) {
-      if (a.epilogue == kEpiResidual)
-        out[t] += v[t];
-      else
-        out[t] = v[t];
-    }
+    if (gn + t < a.N) out[t] = v[t];
   }
 }
 
@@ -1237,34 +1233,45 @@ __global__ void __launch_bounds__(64 * WAVES) gemm_decode_kernel(GemmArgs a, int
 }
 
 // The operand's RMSNorm computed by every workgroup of the projection (GemmArgs::norm), row by
-// row, with Q chunks of four columns per thread: a launch of its own is a chain of two memory
+// row, with Q chunks of eight columns per thread: a launch of its own is a chain of two memory
 // round trips and a kernel boundary, 4 us per norm of one row, and here the weights' first loads
 // (`prefetch`) are in flight behind it. Every workgroup reads the rows and their partials, so it
-// pays for one or two rows only. put(row, column, four halves) stores the operand.
+// pays for one or two rows only. The arithmetic and its order are rmsnorm_flayout_kernel's (chunk
+// c is that kernel's thread c, wave c / 64), so a row does not depend on the pass's other rows.
+// put(row, column, eight halves) stores the operand.
 template <int NT, int Q, typename Prefetch, typename Put>
 __device__ inline void fold_norm_row(const NormFold& f, int row, bool publish, float* scratch, Prefetch&& prefetch,
                                      Put&& put) {
   constexpr int U = 12 / Q;  // partials' loads in flight at once, at clamped addresses
+  constexpr int kWaves = NT / 64;
   const int wave = threadIdx.x >> 6;
-  floatx4 v[Q], w[Q], y[Q];
+  float v[Q][8], w[Q][8], y[Q][8];
   int c[Q], at[Q];
+  const auto load8 = [](const float* src, float* dst) {
+    const floatx4 lo = *reinterpret_cast<const floatx4*>(src), hi = *reinterpret_cast<const floatx4*>(src + 4);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      dst[j] = lo[j];
+      dst[4 + j] = hi[j];
+    }
+  };
 #pragma unroll
   for (int q = 0; q < Q; ++q) {
-    c[q] = 4 * ((int)threadIdx.x + q * NT);
-    at[q] = min(c[q], f.hidden - 4);
-    v[q] = *reinterpret_cast<const floatx4*>(f.h + (size_t)row * f.hidden + at[q]);
-    w[q] = *reinterpret_cast<const floatx4*>(f.weight + at[q]);
-    y[q] = floatx4{0.f, 0.f, 0.f, 0.f};
+    c[q] = 8 * ((int)threadIdx.x + q * NT);
+    at[q] = min(c[q], f.hidden - 8);
+    load8(f.h + (size_t)row * f.hidden + at[q], v[q]);
+    load8(f.weight + at[q], w[q]);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) y[q][j] = 0.0f;
   }
   const float* base = (f.parts > 0 ? f.partials : f.h) + (size_t)row * f.hidden;
-  floatx4 p[U][Q];
+  float p[U][Q][8];
   int s0 = 0;
   const auto load = [&] {
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
-      for (int q = 0; q < Q; ++q)
-        p[u][q] = *reinterpret_cast<const floatx4*>(base + (size_t)max(0, min(s0 + u, f.parts - 1)) * f.stride + at[q]);
+      for (int q = 0; q < Q; ++q) load8(base + (size_t)max(0, min(s0 + u, f.parts - 1)) * f.stride + at[q], p[u][q]);
   };
   const auto sum = [&] {
 #pragma unroll
@@ -1272,7 +1279,7 @@ __device__ inline void fold_norm_row(const NormFold& f, int row, bool publish, f
 #pragma unroll
       for (int q = 0; q < Q; ++q)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) y[q][j] = s0 + u < f.parts ? y[q][j] + p[u][q][j] : y[q][j];
+        for (int j = 0; j < 8; ++j) y[q][j] = s0 + u < f.parts ? y[q][j] + p[u][q][j] : y[q][j];
   };
   load();
   while (s0 + U < f.parts) {
@@ -1282,40 +1289,47 @@ __device__ inline void fold_norm_row(const NormFold& f, int row, bool publish, f
   }
   prefetch();
   sum();
-  float squares = 0.0f;
 #pragma unroll
   for (int q = 0; q < Q; ++q) {
     const bool in = c[q] < f.hidden;
+    if (f.parts > 0) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      v[q][j] += y[q][j];
-      squares += in ? v[q][j] * v[q][j] : 0.0f;
+      for (int j = 0; j < 8; ++j) v[q][j] += y[q][j];
     }
-    if (publish && f.h_out && in) *reinterpret_cast<floatx4*>(f.h_out + (size_t)row * f.hidden + c[q]) = v[q];
+    if (publish && f.h_out && in) {
+      float* dst = f.h_out + (size_t)row * f.hidden + c[q];
+      *reinterpret_cast<floatx4*>(dst) = floatx4{v[q][0], v[q][1], v[q][2], v[q][3]};
+      *reinterpret_cast<floatx4*>(dst + 4) = floatx4{v[q][4], v[q][5], v[q][6], v[q][7]};
+    }
+    float squares = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      v[q][j] = in ? v[q][j] : 0.0f;
+      squares += v[q][j] * v[q][j];
+    }
+    for (int o = 32; o > 0; o >>= 1) squares += __shfl_xor(squares, o, 64);
+    if ((threadIdx.x & 63) == 0) scratch[q * kWaves + wave] = squares;
   }
-  for (int o = 32; o > 0; o >>= 1) squares += __shfl_xor(squares, o, 64);
-  if ((threadIdx.x & 63) == 0) scratch[wave] = squares;
   __syncthreads();
   float total = 0.0f;
 #pragma unroll
-  for (int t = 0; t < NT / 64; ++t) total += scratch[t];
+  for (int t = 0; t < Q * kWaves; ++t) total += scratch[t];
   __syncthreads();
   const float inverse = 1.0f / sqrtf(total / (float)f.hidden + f.eps);
 #pragma unroll
   for (int q = 0; q < Q; ++q) {
     if (c[q] >= f.hidden) continue;
-    half4 x;
+    half8 x;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) x[j] = to_half((v[q][j] * inverse) * w[q][j]);
+    for (int j = 0; j < 8; ++j) x[j] = to_half((v[q][j] * inverse) * w[q][j]);
     put(row, c[q], x);
   }
 }
 
 // gemm_decode_kernel's deferred projection (eight waves of one fragment row, the split's
 // operand whole in LDS) for the one or two rows of a folded RMSNorm.
-template <int Q>
 __global__ void __launch_bounds__(512) gemm_norm_kernel(GemmArgs a, int n_tiles) {
-  constexpr int P = 4;
+  constexpr int P = 4, Q = kFoldHidden / (8 * 512);
   extern __shared__ float lds[];  // the split's fragments [per][64] half8, then 8 floats
   half8* xs = reinterpret_cast<half8*>(lds);
   const int tile_n = blockIdx.x % n_tiles, split = blockIdx.x / n_tiles;
@@ -1328,10 +1342,9 @@ __global__ void __launch_bounds__(512) gemm_norm_kernel(GemmArgs a, int n_tiles)
   const half8* W = reinterpret_cast<const half8*>(a.w_hi) + (size_t)frag * KT * 64 + lane;
   half8 rw[P];
   const auto load_w = [&](int slot, int kt) { rw[slot] = __builtin_nontemporal_load(W + (size_t)min(kt, kt_last) * 64); };
-  const auto put = [&](int row, int c, half4 x) {
+  const auto put = [&](int row, int c, half8 x) {
     const int s = (c >> 5) - kt0;
-    if (s >= 0 && s < steps)
-      *reinterpret_cast<half4*>(reinterpret_cast<_Float16*>(xs + s * 64 + row + ((c & 31) >> 3) * 16) + (c & 7)) = x;
+    if (s >= 0 && s < steps) xs[s * 64 + row + ((c & 31) >> 3) * 16] = x;
   };
   float* scratch = lds + (size_t)per * 256;
   fold_norm_row<512, Q>(
@@ -1374,7 +1387,7 @@ __global__ void __launch_bounds__(512) gemm_norm_kernel(GemmArgs a, int n_tiles)
 template <int MF, int NP, int WK, int P, int Q>
 __global__ void __launch_bounds__(64 * WK) gemm_pair_kernel(GemmArgs a) {
   constexpr int NF = 2 * NP;
-  extern __shared__ float lds[];  // [WK][MF][NF][64] floatx4, then (Q > 0) [kFoldRows][Kp] halves and WK floats
+  extern __shared__ float lds[];  // [WK][MF][NF][64] floatx4, then (Q > 0) [M][Kp] halves and Q * WK floats
   const int M = a.device_m ? *a.device_m : a.M;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int KT = (int)(a.Kp >> 5);
@@ -1421,8 +1434,8 @@ __global__ void __launch_bounds__(64 * WK) gemm_pair_kernel(GemmArgs a) {
   };
   if constexpr (Q > 0) {
     static_assert(MF == 1, "folded rows are one row tile");
-    float* scratch = reinterpret_cast<float*>(xs + (size_t)kFoldRows * a.Kp);
-    const auto put = [&](int row, int c, half4 x) { *reinterpret_cast<half4*>(xs + (size_t)row * a.Kp + c) = x; };
+    float* scratch = reinterpret_cast<float*>(xs + (size_t)M * a.Kp);
+    const auto put = [&](int row, int c, half8 x) { *reinterpret_cast<half8*>(xs + (size_t)row * a.Kp + c) = x; };
     fold_norm_row<64 * WK, Q>(a.norm, 0, blockIdx.x == 0, scratch, fill, put);
     for (int row = 1; row < M; ++row) fold_norm_row<64 * WK, Q>(a.norm, row, blockIdx.x == 0, scratch, [] {}, put);
     __syncthreads();
@@ -1476,14 +1489,14 @@ void launch_pair_shape(hipStream_t stream, const GemmArgs& a) {
   if ((uint64_t)MF * 16 > a.x_rows_padded) fail(HLLM_INTERNAL, "GEMM tile exceeds the activation padding");
   if (a.N % (32 * NP) != 0 || (uint64_t)a.N > a.w_rows_padded) fail(HLLM_INTERNAL, "gate/up pairs exceed the weights");
   constexpr size_t tiles = (size_t)WK * MF * NP * 2 * 1024;
-  constexpr size_t most = tiles + (Q > 0 ? kFoldRows * kFoldHidden * 2 + WK * 4 : 0);
+  constexpr size_t most = tiles + (Q > 0 ? 2 * kFoldHidden + Q * WK * 4 : 0);
   static const bool configured = [] {
     HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_pair_kernel<MF, NP, WK, P, Q>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)most));
     return true;
   }();
   (void)configured;
-  const size_t lds = tiles + (Q > 0 ? kFoldRows * a.Kp * 2 + WK * 4 : 0);
+  const size_t lds = tiles + (Q > 0 ? 2 * a.M * a.Kp + Q * WK * 4 : 0);
   observed(kernel_name<MF, NP, WK, P, Q>("gemm_pair_kernel"),
            [&] { gemm_pair_kernel<MF, NP, WK, P, Q><<<dim3(a.N / (32 * NP)), 64 * WK, lds, stream>>>(a); });
 }
@@ -1747,9 +1760,9 @@ const DecodeShape& decode_shape(bool pair) {
   return pair ? paired : deferred;
 }
 
-// Whether the decode kernel runs this projection: F16, and at most 64 rows where a consumer
-// sums K splits or for SwiGLU (never split), or at most 128 rows with enough output features to
-// fill the GPU unsplit (the LM head: Qwen3-4B's at 128 rows 199 -> 172 us
+// Whether the decode kernel runs this projection: F16, and at most 64 rows where a consumer sums
+// K splits or for SwiGLU (never split), or at most 128 rows with enough output features to fill
+// the GPU unsplit (the LM head: Qwen3-4B's at 128 rows 199 -> 172 us
 // against the activation-staged kernel, 4.5 TB/s).
 bool decode_applies(const GemmArgs& a, int prec, int rows, int cus) {
   const bool summed = a.defer_reduce || a.epilogue == kEpiSwiglu;
@@ -1762,14 +1775,15 @@ bool decode_applies(const GemmArgs& a, int prec, int rows, int cus) {
   return n_tiles * waves >= 4 * cus;
 }
 
-// Whether gate/up runs on the pair kernel: up to 16 rows always, more rows where the decode
-// kernel's workgroups (64 pairs' features each) would leave half of the CUs or more without
-// one. Measured per launch (event times), decode kernel -> pair kernel: Qwen3-0.6B (48
-// workgroups) 10.0 -> 6.8 us at 4 rows, 12.4 -> 7.8 at 48, 13.1 -> 8.5 at 64; 16 384 columns of
-// K 2 048 (128) 19.9 -> 15.0 at 4 rows, 21.7 -> 17.4 at 64; Falcon3-3B (144) 25.8 -> 25.3 at 4
-// rows but 25.1 -> 27.8 at 32; Qwen3-4B (152) 21.6 -> 21.0 at 4 and 24.7 -> 30.3 at 64.
-bool pair_applies(const GemmArgs& a, int rows, int cus) {
-  return a.epilogue == kEpiSwiglu && a.N % 64 == 0 && (rows <= 16 || (a.N + 127) / 128 <= cus / 2);
+// Whether gate/up runs on the pair kernel: where the decode kernel's workgroups (64 pairs'
+// features each) would leave half of the CUs or more without one, for every row count alike, so
+// that a row's sums do not depend on the rows beside it. Measured per launch (event times),
+// decode kernel -> pair kernel: Qwen3-0.6B (48 workgroups) 10.0 -> 6.8 us at 4 rows, 12.4 -> 7.8 at
+// 48, 13.1 -> 8.5 at 64; 16 384 columns of K 2 048 (128) 19.9 -> 15.0 at 4 rows, 21.7 -> 17.4 at 64;
+// Falcon3-3B (144) 25.8 -> 25.3 at 4 rows but 25.1 -> 27.8 at 32; Qwen3-4B (152) 21.6 -> 21.0 at 4
+// and 24.7 -> 30.3 at 64.
+bool pair_applies(const GemmArgs& a, int cus) {
+  return a.epilogue == kEpiSwiglu && a.N % 64 == 0 && (a.N + 127) / 128 <= cus / 2;
 }
 
 // Fragment rows per wave of the unpaired decode variant: the configured count, halved while
@@ -1802,9 +1816,7 @@ int launch_decode_variant(hipStream_t stream, const GemmArgs& a, int cus) {
   const int n_tiles = (a.N + 16 * fr - 1) / (16 * fr);
   int ksplit = 1;
   if (a.defer_reduce) ksplit = decode_splits(chunks, n_tiles, waves, cus);
-  if constexpr (MF > 1) {  // one row tile: the pair kernel
-    if (pair) return launch_decode_waves<MF, 2, KC, P, true, P>(stream, a, waves, 1);
-  }
+  if (pair) return launch_decode_waves<MF, 2, KC, P, true, P>(stream, a, waves, 1);
   if (nfw == 4) return launch_decode_waves<MF, 4, KC, P, false, (PW > 8 ? 8 : PW)>(stream, a, waves, ksplit);
   if (nfw == 2) return launch_decode_waves<MF, 2, KC, P, false, PW>(stream, a, waves, ksplit);
   return launch_decode_waves<MF, 1, KC, P, false, PW>(stream, a, waves, ksplit);
@@ -1836,12 +1848,10 @@ void launch_pair(hipStream_t stream, const GemmArgs& a, int cus) {
 // A projection with its operand's RMSNorm folded in (gemm_folds_norm): returns the partials left.
 int launch_folded(hipStream_t stream, GemmArgs a, int cus) {
   if (a.epilogue == kEpiSwiglu) {
-    switch ((a.norm.hidden + 1023) / 1024) {
-      case 1: launch_pair_shape<1, 1, 4, 4, 1>(stream, a); break;
-      case 2: launch_pair_shape<1, 1, 4, 4, 2>(stream, a); break;
-      case 3: launch_pair_shape<1, 1, 4, 4, 3>(stream, a); break;
-      default: launch_pair_shape<1, 1, 4, 4, 4>(stream, a); break;
-    }
+    if (a.norm.hidden <= 2048)
+      launch_pair_shape<1, 1, 4, 4, 1>(stream, a);
+    else
+      launch_pair_shape<1, 1, 4, 4, 2>(stream, a);
     return 0;
   }
   const int n_tiles = (a.N + 127) / 128, KT = (int)(a.Kp >> 5), chunks = (KT + 3) / 4;
@@ -1850,24 +1860,18 @@ int launch_folded(hipStream_t stream, GemmArgs a, int cus) {
   if ((size_t)a.ksplit * a.M * a.N > a.workspace_floats) a.ksplit = 1;
   const int per = ((KT + a.ksplit - 1) / a.ksplit + 3) / 4 * 4;
   const size_t lds = (size_t)per * 1024 + 8 * sizeof(float);
-  const auto go = [&](auto kernel, const char* name) {
-    static const bool configured = [kernel] {
-      HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    160 * 1024));
-      return true;
-    }();
-    (void)configured;
-    observed(name, [&] { kernel<<<dim3(n_tiles * a.ksplit), 512, lds, stream>>>(a, n_tiles); });
-  };
-  if (a.norm.hidden <= 2048)
-    go(&gemm_norm_kernel<1>, "gemm_norm_kernel<1>");
-  else
-    go(&gemm_norm_kernel<2>, "gemm_norm_kernel<2>");
+  static const bool configured = [] {
+    HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_norm_kernel),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+    return true;
+  }();
+  (void)configured;
+  observed("gemm_norm_kernel", [&] { gemm_norm_kernel<<<dim3(n_tiles * a.ksplit), 512, lds, stream>>>(a, n_tiles); });
   return a.ksplit > 1 ? a.ksplit : 0;
 }
 
 int launch_decode(hipStream_t stream, const GemmArgs& a, int rows, int cus) {
-  if (pair_applies(a, rows, cus)) {
+  if (pair_applies(a, cus)) {
     if (rows <= 16)
       launch_pair<1>(stream, a, cus);
     else if (rows <= 32)
@@ -1906,7 +1910,7 @@ bool gemm_folds_norm(const GemmArgs& a, int prec, int rows, int hidden, int cus)
   if (forced_config().load(std::memory_order_relaxed) >= 0 || env_int("HLLM_ROCM_DECODE_OFF", 0) != 0 ||
       env_int("HLLM_ROCM_DECODE_WHOLE", 1) == 0 || env_int("HLLM_ROCM_NORM_FOLD", 1) == 0)
     return false;
-  return decode_applies(a, prec, rows, cus) && (a.epilogue == kEpiSwiglu ? pair_applies(a, rows, cus) : a.epilogue == kEpiStore && a.defer_reduce != 0);
+  return decode_applies(a, prec, rows, cus) && (a.epilogue == kEpiSwiglu ? pair_applies(a, cus) : a.epilogue == kEpiStore && a.defer_reduce != 0);
 }
 
 int gemm_argmax_parts(const GemmArgs& a, int prec, int rows_bound, int cus) {
