@@ -1760,14 +1760,13 @@ const DecodeShape& decode_shape(bool pair) {
   return pair ? paired : deferred;
 }
 
-// Whether the decode kernel runs this projection: F16, and at most 64 rows where a consumer sums
-// K splits or for SwiGLU (never split), or at most 128 rows with enough output features to fill
-// the GPU unsplit (the LM head: Qwen3-4B's at 128 rows 199 -> 172 us
+// Whether the decode kernels run this projection: F16, and at most 64 rows where a consumer sums
+// K splits, at most 128 rows for SwiGLU (never split; measured at pair_applies) and for outputs
+// with enough features to fill the GPU unsplit (the LM head: Qwen3-4B's at 128 rows 199 -> 172 us
 // against the activation-staged kernel, 4.5 TB/s).
 bool decode_applies(const GemmArgs& a, int prec, int rows, int cus) {
-  const bool summed = a.defer_reduce || a.epilogue == kEpiSwiglu;
-  if (prec != kF16 || rows > (summed ? 64 : 128) || rows <= 0) return false;
-  if (summed) return true;
+  if (prec != kF16 || rows > (a.defer_reduce ? 64 : 128) || rows <= 0) return false;
+  if (a.defer_reduce || a.epilogue == kEpiSwiglu) return true;
   const DecodeShape& d = decode_shape(false);
   const int waves = d.waves >= 8 ? 8 : 4;
   if (rows > 64 && (waves != 8 || d.frags != 1)) return false;  // its only shape above 64 rows
@@ -1781,7 +1780,9 @@ bool decode_applies(const GemmArgs& a, int prec, int rows, int cus) {
 // decode kernel -> pair kernel: Qwen3-0.6B (48 workgroups) 10.0 -> 6.8 us at 4 rows, 12.4 -> 7.8 at
 // 48, 13.1 -> 8.5 at 64; 16 384 columns of K 2 048 (128) 19.9 -> 15.0 at 4 rows, 21.7 -> 17.4 at 64;
 // Falcon3-3B (144) 25.8 -> 25.3 at 4 rows but 25.1 -> 27.8 at 32; Qwen3-4B (152) 21.6 -> 21.0 at 4
-// and 24.7 -> 30.3 at 64.
+// and 24.7 -> 30.3 at 64. 65 to 128 rows ran on the activation-staged kernel before: Qwen3-0.6B at
+// 96 rows 20.2 -> 9.8 us here, 16 384 columns 33.3 -> 20.1; on the decode kernel Qwen3-4B 36.4 -> 29.5
+// at 96 rows and 37.0 -> 36.0 at 128, Falcon3-3B 57.7 -> 33.4 and 57.3 -> 40.8.
 bool pair_applies(const GemmArgs& a, int cus) {
   return a.epilogue == kEpiSwiglu && a.N % 64 == 0 && (a.N + 127) / 128 <= cus / 2;
 }
@@ -1840,7 +1841,7 @@ int launch_decode_rows(hipStream_t stream, const GemmArgs& a, int cus) {
 template <int MF>
 void launch_pair(hipStream_t stream, const GemmArgs& a, int cus) {
   if constexpr (MF > 1) {
-    if (a.N / 32 > cus) return launch_pair_shape<MF, 2, 4, 4>(stream, a);
+    if (a.N / 32 > cus) return launch_pair_shape<MF, 2, 4, (MF > 4 ? 2 : 4)>(stream, a);
   }
   launch_pair_shape<MF, 1, 4, 4>(stream, a);
 }
@@ -1878,14 +1879,22 @@ int launch_decode(hipStream_t stream, const GemmArgs& a, int rows, int cus) {
       launch_pair<2>(stream, a, cus);
     else if (rows <= 48)
       launch_pair<3>(stream, a, cus);
-    else
+    else if (rows <= 64)
       launch_pair<4>(stream, a, cus);
+    else if (rows <= 96)
+      launch_pair<6>(stream, a, cus);
+    else
+      launch_pair<8>(stream, a, cus);
     return 0;
   }
   if (rows <= 16) return launch_decode_rows<1>(stream, a, cus);
   if (rows <= 32) return launch_decode_rows<2>(stream, a, cus);
   if (rows <= 64) return launch_decode_rows<4>(stream, a, cus);
-  return launch_decode_waves<8, 1, 4, 4, false, 4>(stream, a, 8, 1);  // unsplit outputs (decode_applies)
+  // Above 64 rows nothing is split (decode_applies): gate/up pairs in chunks of eight k-steps, two
+  // of which still fit in LDS (chunks of four: 5-10% slower), or plain outputs.
+  if (a.epilogue != kEpiSwiglu) return launch_decode_waves<8, 1, 4, 4, false, 4>(stream, a, 8, 1);
+  if (rows <= 96) return launch_decode_waves<6, 2, 8, 8, true, 8>(stream, a, 4, 1);
+  return launch_decode_waves<8, 2, 8, 8, true, 8>(stream, a, 4, 1);
 }
 
 std::atomic<int>& forced_config() {
