@@ -1912,9 +1912,10 @@ int forced_gemm_config() { return forced_config().load(std::memory_order_relaxed
 
 // (HLLM_ROCM_NORM_FOLD=0, read at every call, says false, for comparisons.)
 bool gemm_folds_norm(const GemmArgs& a, int prec, int rows, int hidden, int cus) {
-  // Every workgroup normalises the rows one after the other: at 2 rows of 2560 and 3072 columns the
-  // passes took 0-2% longer than with separate norms (one row of them 6-7% less; Qwen3-0.6B 573 -> 478
-  // us for one row on fourteen layers and 600 -> 537 for two, 2048 columns 650 -> 575 and 655 -> 627).
+  // Every workgroup normalises the rows one after the other. Separate norms -> folded, us per pass:
+  // one row of Qwen3-0.6B on fourteen layers 552 -> 485, 2048 columns on twelve 640 -> 585, Qwen3-4B on
+  // twelve (q/k/v only) 810 -> 790, Falcon3-3B on six 487 -> 476; two rows 583 -> 560 and 652 -> 645, of
+  // 2560 and 3072 columns no difference (the line is at 2 x 2048).
   if (rows > kFoldRows || rows * hidden > kFoldHidden || (uint64_t)hidden != a.Kp) return false;
   if (forced_config().load(std::memory_order_relaxed) >= 0 || env_int("HLLM_ROCM_DECODE_OFF", 0) != 0 ||
       env_int("HLLM_ROCM_DECODE_WHOLE", 1) == 0 || env_int("HLLM_ROCM_NORM_FOLD", 1) == 0)
