@@ -867,7 +867,11 @@ void run(dim3 grid, int threads, size_t lds, hipStream_t stream, const GemmArgs&
 // output matrices when the consumer sums them.
 int fit_ksplit(const GemmArgs& a, int ksplit, size_t tiles, size_t tile_floats) {
   const size_t need = a.defer_reduce ? (size_t)a.M * a.N : tiles * tile_floats;
-  return (size_t)ksplit * need > a.workspace_floats ? 1 : ksplit;
+  if ((size_t)ksplit * need > a.workspace_floats) ksplit = 1;
+  // The reduce kernel stores its sums; only the unsplit epilogues add to the residual stream.
+  if (ksplit > 1 && a.epilogue == kEpiResidual && !a.defer_reduce)
+    fail(HLLM_INTERNAL, "a residual projection splits K only for a consumer that sums its partials");
+  return ksplit;
 }
 
 template <int MF, int NF, int WM, int WN, int WK, int P>

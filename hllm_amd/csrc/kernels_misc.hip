@@ -290,8 +290,9 @@ __global__ void __launch_bounds__(1024) rmsnorm_flayout_kernel(
 #pragma unroll
     for (int q = 0; q < Q; ++q) load8_at(x + c[q], v[q]);
     if (residual.parts > 0) {
-      // The projection's K-split partials summed in split order from zero, then the
-      // residual add (the order of the reduce kernel's residual epilogue), written back.
+      // The projection's K-split partials summed in split order from zero, then added to the
+      // residual row (the same order as residual_sum_kernel and the boundary's encoding),
+      // written back.
       float y[Q][8];
 #pragma unroll
       for (int q = 0; q < Q; ++q)

@@ -1,0 +1,70 @@
+// Host-side checks of the projection launchers (gemm.hpp): decisions and refusals that are made
+// before any launch, so they need no GPU. Usage: <program> <case>; prints PASS or the reason.
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <string>
+
+#include "gemm.hpp"
+
+using namespace hllm_rocm;
+
+namespace {
+
+constexpr int kCus = 256;
+
+GemmArgs projection(int rows, int n, uint64_t k, int epilogue, bool deferred) {
+  GemmArgs a{};
+  a.M = rows;
+  a.N = n;
+  a.Kp = pad32(k);
+  a.w_rows_padded = (uint64_t)(n + 255) / 256 * 256;
+  a.x_rows_padded = gemm_padded_rows((uint64_t)rows);
+  a.workspace_floats = 32ull << 20;
+  a.epilogue = epilogue;
+  a.defer_reduce = deferred ? 1 : 0;
+  return a;
+}
+
+// The message of the failure that `call` raises before (or instead of) its launch.
+template <typename F>
+std::string failure(F&& call) {
+  try {
+    call();
+  } catch (const Failure& e) {
+    return e.what();
+  }
+  return "";
+}
+
+// A split residual projection without a consumer for its partials is refused by every launcher
+// (the reduce kernel stores its sums, it does not add them to the residual stream).
+bool split_residual_is_refused() {
+  const GemmArgs a = projection(96, 1024, 4096, kEpiResidual, false);
+  for (int config : {0, 9, 12, 15, 16, 18}) {
+    const std::string message = failure([&] { launch_gemm_config(nullptr, a, kF16, a.M, kCus, config, 4); });
+    if (message.find("splits K only for a consumer") == std::string::npos) {
+      std::printf("config %d: '%s'\n", config, message.c_str());
+      return false;
+    }
+  }
+  return true;
+}
+
+struct Case {
+  const char* name;
+  bool (*run)();
+};
+const Case kCases[] = {{"split_residual_is_refused", split_residual_is_refused}};
+
+}  // namespace
+
+int main(int argc, char** argv) {
+  for (const Case& c : kCases) {
+    if (argc > 1 && std::strcmp(argv[1], c.name) != 0) continue;
+    const bool ok = c.run();
+    std::printf("%s %s\n", ok ? "PASS" : "FAIL", c.name);
+    return ok ? 0 : 1;
+  }
+  return 2;
+}

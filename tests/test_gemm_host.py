@@ -1,0 +1,30 @@
+"""What the projection launchers decide and refuse on the host, before any launch
+(tests/host/gemm_host_tests.hip, host code only, against the built libhllm_rocm.so)."""
+import os
+import subprocess
+
+import pytest
+
+from hllm_amd import build
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+@pytest.fixture(scope="module")
+def program():
+    out = os.path.join(build.HERE, "_build", "gemm_host_tests")
+    r = subprocess.run([build.HIPCC, "--offload-host-only", "-O1", "-std=c++17", f"-I{os.path.join(ROOT, 'include')}",
+                        f"-I{build.CSRC}", os.path.join(ROOT, "tests", "host", "gemm_host_tests.hip"), "-o", out + ".tmp",
+                        f"-L{build.HERE}", "-lhllm_rocm", "-Wl,-rpath,$ORIGIN/.."], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout + r.stderr
+    os.replace(out + ".tmp", out)
+    return out
+
+
+def run(program, case, **env):
+    r = subprocess.run([program, case], capture_output=True, text=True, timeout=60, env=dict(os.environ, **env))
+    assert r.returncode == 0 and f"PASS {case}" in r.stdout, r.stdout + r.stderr
+
+
+def test_split_residual_without_a_consumer_is_refused(program):
+    run(program, "split_residual_is_refused")
