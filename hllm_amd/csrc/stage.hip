@@ -327,15 +327,17 @@ class Stage {
   // launches, set the pace). Every launch parameter of a pass is a function of its shape:
   // items, rows, sampled rows, sampler, attention work items and splits, and the host-side
   // choices made per pass (the LM head's argmax-epilogue parts, the forced GEMM
-  // configuration); all other per-pass values are read on the device. A shape is captured
+  // configuration, the norms folded into q/k/v and gate+up); all other per-pass values are
+  // read on the device. A shape is captured
   // the second time it is seen (the first run sets the kernels' attributes eagerly).
   struct PassShape {
     uint32_t items, rows, samples, sampler, attention_items, any_split;
     int32_t argmax_parts, gemm_config;
+    bool fold_qkv, fold_gate_up;
     bool operator<(const PassShape& o) const {
-      return std::tie(items, rows, samples, sampler, attention_items, any_split, argmax_parts, gemm_config) <
-             std::tie(o.items, o.rows, o.samples, o.sampler, o.attention_items, o.any_split, o.argmax_parts,
-                      o.gemm_config);
+      return std::tie(items, rows, samples, sampler, attention_items, any_split, argmax_parts, gemm_config, fold_qkv,
+                      fold_gate_up) < std::tie(o.items, o.rows, o.samples, o.sampler, o.attention_items, o.any_split,
+                                               o.argmax_parts, o.gemm_config, o.fold_qkv, o.fold_gate_up);
     }
   };
   struct CapturedPass {
@@ -1537,7 +1539,7 @@ void Stage::submit(const hllm_rocm_pass& pass, bool phases) {
   try {
     if (phases) HIP_CHECK(hipEventRecord(phase_start_, stream_));
     const PassShape shape{n, (uint32_t)R, (uint32_t)S, sampler ? 1u : 0u, (uint32_t)attn_grid,
-                          attn_any_split ? 1u : 0u, fused_parts, forced_gemm_config()};
+                          attn_any_split ? 1u : 0u, fused_parts, forced_gemm_config(), fold_qkv, fold_gate_up};
     const bool graphable = graphs_enabled_ && !profiling_ && !phases && !pass.logits && !pass.trace_hidden;
     auto found = graphable ? graphs_.find(shape) : graphs_.end();
     if (found != graphs_.end()) {

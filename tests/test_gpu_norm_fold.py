@@ -50,3 +50,30 @@ def test_folded_norms_match_the_oracle(hidden, intermediate, final):
         for s in seqs:
             st.release(s)
     st.close()
+
+
+def test_switch_is_part_of_a_captured_pass(monkeypatch):
+    """With graphs enabled, a pass with HLLM_ROCM_NORM_FOLD=0 does not replay the folded pass's
+    graph, nor the other way round, and every pass returns the bits of an eager stage."""
+    shape = synthetic.ModelShape("graphs", 2, 1024, 1600, 4, 2, 64, VOCAB, eps=1e-6, theta=1e4, qk_norm=False,
+                                 tied=False, max_seq=64)
+    ids = np.random.default_rng(3).integers(0, VOCAB, 7).astype(np.uint64)
+    stages = []
+    for graphs in (False, True):
+        st = capi.Stage(model.stage_config(shape, 0, 1, first=True, final=False, execution="f16",
+                                           kv_cache_bytes=16 << 20, max_sequences=4, max_pass_rows=64))
+        model.synthesize(st, shape, seed=5, norm_sigma=0.1)
+        st.set_graphs(graphs)
+        stages.append((st, st.allocate(len(ids))))
+    stats = []
+    for position, fold in enumerate("1110011"):
+        hp.say("graphs", "position", position, "fold", fold)
+        monkeypatch.setenv("HLLM_ROCM_NORM_FOLD", fold)
+        eager, replayed = [st.execute([capi.item(seq, 1, position, sample=False)],
+                                      token_ids=ids[position:position + 1])["boundary"] for st, seq in stages]
+        assert np.array_equal(eager, replayed), position
+        stats.append(stages[1][0].graph_stats())
+    # (captured, replayed): folded eager, captured, replayed; unfolded eager, captured; folded replayed.
+    assert stats == [(0, 0), (1, 1), (1, 2), (1, 2), (2, 3), (2, 4), (2, 5)], stats
+    for st, _ in stages:
+        st.close()
