@@ -1924,7 +1924,12 @@ bool gemm_folds_norm(const GemmArgs& a, int prec, int rows, int hidden, int cus)
   if (forced_config().load(std::memory_order_relaxed) >= 0 || env_int("HLLM_ROCM_DECODE_OFF", 0) != 0 ||
       env_int("HLLM_ROCM_DECODE_WHOLE", 1) == 0 || env_int("HLLM_ROCM_NORM_FOLD", 1) == 0)
     return false;
-  return decode_applies(a, prec, rows, cus) && (a.epilogue == kEpiSwiglu ? pair_applies(a, cus) : a.epilogue == kEpiStore && a.defer_reduce != 0);
+  if (!decode_applies(a, prec, rows, cus)) return false;
+  if (a.epilogue == kEpiSwiglu) return pair_applies(a, cus);
+  // gemm_norm_kernel has the decode kernel's default launch shape only: with another one its K
+  // splits, and with them a row's sums, would differ from those of three rows.
+  const DecodeShape& d = decode_shape(false);
+  return a.epilogue == kEpiStore && a.defer_reduce != 0 && d.waves >= 8 && d.chunk <= 4 && decode_frags(a, 8) == 1;
 }
 
 int gemm_argmax_parts(const GemmArgs& a, int prec, int rows_bound, int cus) {

@@ -51,11 +51,25 @@ bool split_residual_is_refused() {
   return true;
 }
 
+// q/k/v and gate+up of one row fold their RMSNorm.
+bool folds(bool expect_qkv, bool expect_gate_up) {
+  const bool qkv = gemm_folds_norm(projection(1, 4096, 1024, kEpiStore, true), kF16, 1, 1024, kCus);
+  const bool gate_up = gemm_folds_norm(projection(1, 6144, 1024, kEpiSwiglu, false), kF16, 1, 1024, kCus);
+  if (qkv != expect_qkv || gate_up != expect_gate_up) std::printf("q/k/v folds: %d, gate+up: %d\n", qkv, gate_up);
+  return qkv == expect_qkv && gate_up == expect_gate_up;
+}
+bool norms_fold() { return folds(true, true); }
+// Under a decode launch shape other than the folded kernel's (set in the environment by the caller)
+// q/k/v keeps its separate norm.
+bool another_decode_shape_keeps_the_norm() { return folds(false, true); }
+
 struct Case {
   const char* name;
   bool (*run)();
 };
-const Case kCases[] = {{"split_residual_is_refused", split_residual_is_refused}};
+const Case kCases[] = {{"split_residual_is_refused", split_residual_is_refused},
+                       {"norms_fold", norms_fold},
+                       {"another_decode_shape_keeps_the_norm", another_decode_shape_keeps_the_norm}};
 
 }  // namespace
 

@@ -28,3 +28,11 @@ def run(program, case, **env):
 
 def test_split_residual_without_a_consumer_is_refused(program):
     run(program, "split_residual_is_refused")
+
+
+def test_norms_fold_under_the_default_decode_shape_only(program):
+    """The folded q/k/v kernel splits K as the decode kernel's default launch shape does, so one- and
+    two-row passes fold there alone: otherwise a row's sums would depend on the rows beside it."""
+    run(program, "norms_fold")
+    for shape in ({"HLLM_ROCM_DECODE_WAVES": "4"}, {"HLLM_ROCM_DECODE_FRAGS": "2"}, {"HLLM_ROCM_DECODE_CHUNK": "8"}):
+        run(program, "another_decode_shape_keeps_the_norm", **shape)
