@@ -1914,22 +1914,31 @@ int set_forced_gemm_config(int config) { return forced_config().exchange(config)
 
 int forced_gemm_config() { return forced_config().load(std::memory_order_relaxed); }
 
-// (HLLM_ROCM_NORM_FOLD=0, read at every call, says false, for comparisons.)
-bool gemm_folds_norm(const GemmArgs& a, int prec, int rows, int hidden, int cus) {
+namespace {
+
+// What the folded kernels take, whatever the switches say.
+bool fold_applies(const GemmArgs& a, int prec, int rows, int hidden, int cus) {
   // Every workgroup normalises the rows one after the other. Separate norms -> folded, us per pass:
   // one row of Qwen3-0.6B on fourteen layers 552 -> 485, 2048 columns on twelve 640 -> 585, Qwen3-4B on
   // twelve (q/k/v only) 810 -> 790, Falcon3-3B on six 487 -> 476; two rows 583 -> 560 and 652 -> 645, of
   // 2560 and 3072 columns no difference (the line is at 2 x 2048).
   if (rows > kFoldRows || rows * hidden > kFoldHidden || (uint64_t)hidden != a.Kp) return false;
-  if (forced_config().load(std::memory_order_relaxed) >= 0 || env_int("HLLM_ROCM_DECODE_OFF", 0) != 0 ||
-      env_int("HLLM_ROCM_DECODE_WHOLE", 1) == 0 || env_int("HLLM_ROCM_NORM_FOLD", 1) == 0)
-    return false;
   if (!decode_applies(a, prec, rows, cus)) return false;
   if (a.epilogue == kEpiSwiglu) return pair_applies(a, cus);
   // gemm_norm_kernel has the decode kernel's default launch shape only: with another one its K
   // splits, and with them a row's sums, would differ from those of three rows.
   const DecodeShape& d = decode_shape(false);
   return a.epilogue == kEpiStore && a.defer_reduce != 0 && d.waves >= 8 && d.chunk <= 4 && decode_frags(a, 8) == 1;
+}
+
+}  // namespace
+
+// (HLLM_ROCM_NORM_FOLD=0, read at every call, says false, for comparisons.)
+bool gemm_folds_norm(const GemmArgs& a, int prec, int rows, int hidden, int cus) {
+  if (forced_config().load(std::memory_order_relaxed) >= 0 || env_int("HLLM_ROCM_DECODE_OFF", 0) != 0 ||
+      env_int("HLLM_ROCM_DECODE_WHOLE", 1) == 0 || env_int("HLLM_ROCM_NORM_FOLD", 1) == 0)
+    return false;
+  return fold_applies(a, prec, rows, hidden, cus);
 }
 
 int gemm_argmax_parts(const GemmArgs& a, int prec, int rows_bound, int cus) {
@@ -1945,7 +1954,9 @@ int launch_gemm(hipStream_t stream, const GemmArgs& args, int prec, int rows_bou
   if (rows_bound <= 0) return 0;
   const int forced = forced_config().load(std::memory_order_relaxed);
   if (args.norm.h) {
-    if (!gemm_folds_norm(args, prec, rows_bound, args.norm.hidden, cus)) fail(HLLM_INTERNAL, "the projection cannot fold its norm");
+    // The caller decided (gemm_folds_norm) and has no other operand: a switch that another thread
+    // changes while the pass is enqueued does not take the decision back.
+    if (!fold_applies(args, prec, rows_bound, args.norm.hidden, cus)) fail(HLLM_INTERNAL, "the projection cannot fold its norm");
     return launch_folded(stream, args, cus);
   }
   if (args.epilogue == kEpiArgmax) {

@@ -1,5 +1,6 @@
 // Host-side checks of the projection launchers (gemm.hpp): decisions and refusals that are made
-// before any launch, so they need no GPU. Usage: <program> <case>; prints PASS or the reason.
+// before any launch, so they need no GPU. Operands are placeholders: the program refuses to run
+// where a device is visible. Usage: <program> <case>; prints PASS or the reason.
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -63,17 +64,42 @@ bool norms_fold() { return folds(true, true); }
 // q/k/v keeps its separate norm.
 bool another_decode_shape_keeps_the_norm() { return folds(false, true); }
 
+// A pass decides once whether its norms fold; a configuration forced by another thread before the
+// launch does not fail it. (Without a GPU the launch itself fails, with the runtime's message.)
+bool forced_configuration_keeps_the_decision() {
+  const float row = 0.0f;
+  for (GemmArgs a : {projection(1, 4096, 1024, kEpiStore, true), projection(1, 6144, 1024, kEpiSwiglu, false)}) {
+    if (!gemm_folds_norm(a, kF16, 1, 1024, kCus)) return false;
+    a.norm.h = &row;
+    a.norm.hidden = 1024;
+    set_forced_gemm_config(12);
+    const std::string message = failure([&] { launch_gemm(nullptr, a, kF16, 1, kCus); });
+    set_forced_gemm_config(-1);
+    if (message.find("cannot fold") != std::string::npos) {
+      std::printf("'%s'\n", message.c_str());
+      return false;
+    }
+  }
+  return true;
+}
+
 struct Case {
   const char* name;
   bool (*run)();
 };
 const Case kCases[] = {{"split_residual_is_refused", split_residual_is_refused},
                        {"norms_fold", norms_fold},
-                       {"another_decode_shape_keeps_the_norm", another_decode_shape_keeps_the_norm}};
+                       {"another_decode_shape_keeps_the_norm", another_decode_shape_keeps_the_norm},
+                       {"forced_configuration_keeps_the_decision", forced_configuration_keeps_the_decision}};
 
 }  // namespace
 
 int main(int argc, char** argv) {
+  int devices = 0;
+  if (hipGetDeviceCount(&devices) == hipSuccess && devices > 0) {
+    std::printf("%d devices visible: run with HIP_VISIBLE_DEVICES=-1\n", devices);
+    return 3;
+  }
   for (const Case& c : kCases) {
     if (argc > 1 && std::strcmp(argv[1], c.name) != 0) continue;
     const bool ok = c.run();

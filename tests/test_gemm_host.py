@@ -22,7 +22,8 @@ def program():
 
 
 def run(program, case, **env):
-    r = subprocess.run([program, case], capture_output=True, text=True, timeout=60, env=dict(os.environ, **env))
+    r = subprocess.run([program, case], capture_output=True, text=True, timeout=60,
+                       env=dict(os.environ, HIP_VISIBLE_DEVICES="-1", **env))
     assert r.returncode == 0 and f"PASS {case}" in r.stdout, r.stdout + r.stderr
 
 
@@ -36,3 +37,9 @@ def test_norms_fold_under_the_default_decode_shape_only(program):
     run(program, "norms_fold")
     for shape in ({"HLLM_ROCM_DECODE_WAVES": "4"}, {"HLLM_ROCM_DECODE_FRAGS": "2"}, {"HLLM_ROCM_DECODE_CHUNK": "8"}):
         run(program, "another_decode_shape_keeps_the_norm", **shape)
+
+
+def test_a_configuration_forced_meanwhile_does_not_fail_a_pass(program):
+    """set_gemm_config is process-wide: called by another thread between a pass's decision to fold
+    and its launches, it used to fail the pass and its sequences."""
+    run(program, "forced_configuration_keeps_the_decision")
