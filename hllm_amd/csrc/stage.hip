@@ -509,9 +509,9 @@ Stage::Stage(const hllm_rocm_stage_config& c) : c_(c) {
   HIP_CHECK(hipMemsetAsync(gemm_counters_.ptr, 0, gemm_counters_.bytes, stream_));
   if (c.final_stage) {
     logits_.allocate(items_max_ * V_ * sizeof(float), "logits");
-    // Candidates of the argmax kernels, or of the LM head's argmax epilogue (at most 64 rows,
-    // one candidate per 64 or more features).
-    argmax_capacity_ = std::max<uint64_t>(items_max_ * kArgmaxParts, 64 * ((V_ + 63) / 64));
+    // Candidates of the argmax kernels, or of the LM head's argmax epilogue: one per row and 128
+    // features for at most 128 rows (or per 64 features for at most 64 rows, which is less).
+    argmax_capacity_ = std::max<uint64_t>(items_max_ * kArgmaxParts, 128 * ((V_ + 127) / 128));
     argmax_val_.allocate(argmax_capacity_ * sizeof(float), "argmax");
     argmax_idx_.allocate(argmax_capacity_ * sizeof(int32_t), "argmax");
     sample_blocks_ = (int)std::min<uint64_t>(items_max_, kSampleBlocks);

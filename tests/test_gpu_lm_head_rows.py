@@ -48,3 +48,30 @@ def test_head_of_65_to_128_rows():
         greedy = run(logits=False)
         assert np.array_equal(greedy["tokens"].astype(np.int64), out["logits"].argmax(1))
     st.close()
+
+
+def test_fused_argmax_of_128_rows_with_a_ragged_last_tile():
+    """A vocabulary with 32 features in its last 128-feature tile: the candidates of 128 greedy rows fit,
+    so the passes keep the argmax epilogue (no logits, no argmax_partial_kernel) up to 128 rows."""
+    shape = synthetic.ModelShape("head-ragged", 1, 96, 64, 4, 2, 64, 128 * 128 + 32, eps=1e-6, theta=1e4, qk_norm=False,
+                                 tied=False, max_seq=128)
+    st = capi.Stage(model.stage_config(shape, execution="f16", kv_cache_bytes=16 << 20, max_sequences=128,
+                                       max_pass_rows=128))
+    model.synthesize(st, shape, seed=5, norm_sigma=0.1)
+    ids = np.random.default_rng(3).integers(0, shape.vocab, 128).astype(np.uint64)
+    tokens = {}
+    for logits in (True, False):
+        hp.say(shape.name, "logits", logits)
+        seqs = [st.allocate(1) for _ in range(128)]
+        st.profile("argmax")
+        out = st.execute([capi.item(s, 1, 0) for s in seqs], token_ids=ids, want_logits=logits)
+        kernels = [r for r in st.profile_records() if r.startswith("argmax/")]
+        st.profile(None)
+        assert ("argmax/argmax_partial_kernel" in kernels) == logits, kernels
+        tokens[logits] = out["tokens"].astype(np.int64)
+        if logits:
+            assert np.array_equal(tokens[True], out["logits"].argmax(1))
+        for s in seqs:
+            st.release(s)
+    assert np.array_equal(tokens[True], tokens[False])
+    st.close()
