@@ -1621,18 +1621,17 @@ int deferred_splits(int rows, int n, int kt) {
   return std::min({std::max(1, (int)(280.0 / tiles + 0.5)), 8, std::max(1, kt / 8)});
 }
 
-// Tile height and K split of F16 passes of 224 rows and more, by the estimated time: rounds of
-// workgroups over the fullest XCD's CUs (xcd_tile), times the k-steps of a split, times the
-// tile's time per k-step, plus the partials (written here and read back by the consumer, 8
-// bytes per output and split, at about 4.5 TB/s). The times per k-step are those of one round
-// of the Qwen3-4B and Falcon3-3B projections: LDS-copy tiles of 128, 192 and 256 rows 0.51, 0.72
-// and 0.90 us (one workgroup per CU; bound by the copies, so a taller tile is cheaper per
-// row), and activation-staged 128-row tiles 0.8 us with two workgroups per CU (1.0 us in the
-// only round). Measured per layer against the earlier choice by row ranges (all
-// above 768 rows on activation-staged tiles): Falcon3-3B at 1300 rows, q/k/v 77 -> 50, o 45 -> 41,
-// gate+up 164 -> 139, down 112 -> 82 us; Qwen3-4B at 1024 rows 55 -> 44, 42 -> 31, 120 -> 116, 76 ->
-// 54 us; gate+up of Qwen3-0.6B at 512 rows (a K split and a reduce kernel before) 31 -> 23 us.
-Choice tile_choice(int rows, int n, uint64_t kp, bool deferred, size_t workspace_floats, int cus) {
+// Tile height and K split of F16 projections of 224 rows and more whose consumer sums the partials,
+// by the estimated time: rounds of workgroups over the fullest XCD's CUs (xcd_tile), times the
+// k-steps of a split, times the tile's time per k-step, plus the partials (written here and read
+// back by the consumer, 8 bytes per output and split, at about 4.5 TB/s). The times per k-step are
+// those of one round of the Qwen3-4B and Falcon3-3B projections: LDS-copy tiles of 128, 192 and
+// 256 rows 0.51, 0.72 and 0.90 us (one workgroup per CU; bound by the copies, so a taller tile is
+// cheaper per row), and activation-staged 128-row tiles 0.8 us with two workgroups per CU (1.0 us in
+// the only round). Measured per layer against the earlier choice by row ranges (all above 768 rows
+// on activation-staged tiles): Falcon3-3B at 1300 rows, q/k/v 77 -> 50, o 45 -> 41, down 112 -> 82 us;
+// Qwen3-4B at 1024 rows 55 -> 44, 42 -> 31, 76 -> 54 us.
+Choice tile_choice(int rows, int n, uint64_t kp, size_t workspace_floats, int cus) {
   struct Tile {
     int config, bm, per_cu;
     double step_us, only_round_us;
@@ -1644,17 +1643,58 @@ Choice tile_choice(int rows, int n, uint64_t kp, bool deferred, size_t workspace
   // Above 1536 rows (there the row tiles alone fill the CUs on most shapes) the K split is that
   // of 280 workgroups of 128-row tiles, as for F32 execution: full passes of long prompts keep
   // their order of summation, and with it the tokens at near ties, whatever tile runs them.
-  const int kept = rows > 1536 && deferred ? deferred_splits(rows, n, kt) : 0;
+  const int kept = rows > 1536 ? deferred_splits(rows, n, kt) : 0;
   Choice best{15, 1};
   double least = 1e30;
   for (const Tile& t : kTiles) {
     const int m_tiles = (rows + t.bm - 1) / t.bm, slots = std::max(1, cus / kXcds) * t.per_cu;
-    const int most = kept > 0 ? kept : deferred && t.per_cu == 1 ? 8 : 1;
+    const int most = kept > 0 ? kept : t.per_cu == 1 ? 8 : 1;
     for (int ks = std::max(1, kept); ks <= most; ++ks) {
       if (ks > 1 && kept == 0 && (kt / ks < 12 || (size_t)ks * rows * n > workspace_floats)) break;
       const int rounds = ((n_tiles * ks + kXcds - 1) / kXcds * m_tiles + slots - 1) / slots;
       const double steps_us = (kt + ks - 1) / ks * (rounds == 1 ? t.only_round_us : rounds * t.step_us);
-      const double us = steps_us + (deferred ? ks * partial_us : 0.0);
+      const double us = steps_us + ks * partial_us;
+      if (us < least) {
+        least = us;
+        best = {t.config, ks};
+      }
+    }
+  }
+  return best;
+}
+
+// Tile and K split of a many-row projection without a consumer for its partials (gate/up, LM head),
+// by the estimated time: a fixed part, the k-steps of a split times the time per k-step while no CU
+// of the fullest XCD (xcd_tile) has more than one workgroup (only_us) or at that many workgroups per
+// CU (per_us), and for a split the reduce kernel (5 us and the padded partials written and read,
+// 8 bytes each, at 4.7 TB/s). The figures are fitted to event times of every tile and split on
+// sixteen gate/up shapes (512 to 19 456 columns of K 512 to 8192) at 224 to 2048 rows; the tile
+// taken is within 4% of the best of the earlier rules' on all of them. Wide projections stay
+// unsplit (Falcon3-3B's gate+up at 1300 rows 164 us by row ranges, 143 now; Qwen3-0.6B's at 512
+// rows 32 and 17.6), narrow ones need the splits or the small tile to fill the chip: 2048 columns of K 4096 at
+// 224 rows 59 us on unsplit 128-row tiles, 23 split eight ways; K 8192 111 and 28 us; 3072
+// columns of K 2048 34.6 and 24; an LM head of 2000 features of K 2560 at 224 rows 41 and 21 us.
+struct TimedTile {
+  int config, bm, most_splits, least_steps;
+  double fixed_us, only_us, per_us;
+};
+constexpr TimedTile kF16Tiles[] = {{12, 64, 16, 16, 8.3, 0.33, 0.275}, {9, 128, 16, 8, 10.5, 0.50, 0.40},
+                                   {15, 128, 1, 12, 11.0, 0.42, 0.51}, {18, 192, 1, 10, 14.0, 0.58, 0.69},
+                                   {16, 256, 1, 10, 15.5, 0.70, 0.87}};
+template <size_t N>
+Choice timed_choice(const TimedTile (&tiles)[N], int rows, int n, uint64_t kp, size_t workspace_floats, int cus) {
+  const int n_tiles = (n + 255) / 256, kt = (int)(kp >> 5), per_xcd = std::max(1, cus / kXcds);
+  Choice best{tiles[0].config, 1};
+  double least = 1e30;
+  for (const TimedTile& t : tiles) {
+    const int m_tiles = (rows + t.bm - 1) / t.bm, most = std::max(1, std::min(t.most_splits, kt / t.least_steps));
+    const double partials = (double)m_tiles * t.bm * n_tiles * 256;  // per split
+    for (int want = 1, last = 0; last < most; want *= 2) {
+      const int ks = last = std::min(want, most);
+      if (ks > 1 && ks * partials > (double)workspace_floats) break;
+      const int load = ((n_tiles * ks + kXcds - 1) / kXcds * m_tiles + per_xcd - 1) / per_xcd;
+      const double us = t.fixed_us + (kt + ks - 1) / ks * (load == 1 ? t.only_us : load * t.per_us) +
+                        (ks > 1 ? 5.0 + 8.0 * ks * partials / 4.7e6 : 0.0);
       if (us < least) {
         least = us;
         best = {t.config, ks};
@@ -1669,7 +1709,8 @@ Choice tile_choice(int rows, int n, uint64_t kp, bool deferred, size_t workspace
 //  - up to 64 rows: the register-streaming kernels (BM 16/32/64), except for very wide outputs
 //    (gate+up, LM head) with more than 32 rows, where staging the activations in LDS once per
 //    256-feature tile wins;
-//  - F16 passes from 224 rows: tile_choice; F32 execution by the size of the weights;
+//  - F16 passes from 224 rows: tile_choice where the consumer sums the partials, else
+//    timed_choice; F32 execution by the size of the weights;
 //  - the rest: the activation-staged kernel, BM 64, or BM 128 from 384 rows.
 // K is split while there are few output tiles. When the consumer sums the partials
 // (`deferred`) a split costs one partial write, so about 220-280 workgroups are targeted;
@@ -1678,7 +1719,9 @@ Choice tile_choice(int rows, int n, uint64_t kp, bool deferred, size_t workspace
 Choice gemm_choice(int rows, int n, uint64_t kp, bool deferred, bool f16, size_t workspace_floats, int cus) {
   const bool wide = n >= 16384;
   const auto rounded = [](double x) { return std::max(1, (int)(x + 0.5)); };
-  if (f16 && rows >= 224) return tile_choice(rows, n, kp, deferred, workspace_floats, cus);
+  if (f16 && rows >= 224)
+    return deferred ? tile_choice(rows, n, kp, workspace_floats, cus)
+                    : timed_choice(kF16Tiles, rows, n, kp, workspace_floats, cus);
   if (f16 && deferred && rows > 64) {
     // 65-223 rows: 64-row activation-staged tiles (at least two chunks per split), or the
     // 128-row LDS-copy tiles where they allow more than twice the K splits (less work per
