@@ -1716,7 +1716,8 @@ Choice timed_choice(const TimedTile (&tiles)[N], int rows, int n, uint64_t kp, s
 // (`deferred`) a split costs one partial write, so about 220-280 workgroups are targeted;
 // otherwise a reduce kernel reads every partial back, so splits stop at about 200
 // workgroups, in powers of two.
-Choice gemm_choice(int rows, int n, uint64_t kp, bool deferred, bool f16, size_t workspace_floats, int cus) {
+Choice gemm_choice(int rows, int n, uint64_t kp, bool deferred, int prec, size_t workspace_floats, int cus) {
+  const bool f16 = prec == kF16;
   const bool wide = n >= 16384;
   const auto rounded = [](double x) { return std::max(1, (int)(x + 0.5)); };
   if (f16 && rows >= 224)
@@ -1749,14 +1750,16 @@ Choice gemm_choice(int rows, int n, uint64_t kp, bool deferred, bool f16, size_t
   }
   if (!f16) {
     // F32 execution (split activations, two or three products per weight fragment): 16-row
-    // register-streaming tiles while their repeated weight reads stay small (the weights once
-    // per 16 rows, from L2), the activation-staged kernel's 32-row tiles from 224 to 1024 rows
-    // (128-row tiles win at 2048: 1177 / 1031 us per Qwen3-4B layer). Qwen3-0.6B
-    // at 96 rows against 64-row tiles: q/k/v 16.6 -> 10.6, o 15.2 -> 8.5, gate+up 24.4 -> 14.6, down
-    // 16.0 -> 9.2 us; at 120 MB the two meet (q/k/v 16.0 / 16.4 us at 224 rows; 157 MB of Qwen3-4B's
-    // at 65 rows 21.3 / 18.3). 32-row tiles, Qwen3-4B at 512 rows: 67 -> 47, 53 -> 38, 160 -> 119, 96 -> 74
-    // us per projection, at 224 rows 44 -> 30, 37 -> 24, 81 -> 73, 58 -> 44.
-    const double tile_reads = (rows + 15) / 16 * 2.0 * n * (double)kp;
+    // register-streaming tiles while their repeated weight reads stay small (the weights, two
+    // bytes each or four resident as F32, once per 16 rows, from L2), the activation-staged kernel's
+    // 32-row tiles from 224 to 1024 rows (128-row tiles win at 2048: 1177 / 1031 us per
+    // Qwen3-4B layer). Qwen3-0.6B at 96 rows against 64-row tiles: q/k/v 16.6 -> 10.6, o 15.2 -> 8.5,
+    // gate+up 24.4 -> 14.6, down 16.0 -> 9.2 us; at 120 MB the two meet (q/k/v 16.0 / 16.4 us at 224
+    // rows; 157 MB of Qwen3-4B's at 65 rows 21.3 / 18.3; F32-resident, past the line at 223 rows,
+    // q/k/v 23.0 / 19.7 us and, at 65 rows, Qwen3-4B's o 26.7 / 21.8). 32-row tiles, Qwen3-4B at 512 rows:
+    // 67 -> 47, 53 -> 38, 160 -> 119, 96 -> 74 us per projection, at 224 rows 44 -> 30, 37 -> 24, 81 -> 73,
+    // 58 -> 44.
+    const double tile_reads = (rows + 15) / 16 * (prec == kSplitAB ? 4.0 : 2.0) * n * (double)kp;
     if (tile_reads <= 120e6) return {0, 0};
     if (rows >= 224 && rows <= 1024) return {11, deferred ? 0 : 1};
   }
@@ -2012,8 +2015,7 @@ int launch_gemm(hipStream_t stream, const GemmArgs& args, int prec, int rows_bou
     return launch_decode(stream, args, rows_bound, cus);
   if (forced == kDecodeConfig && prec == kF16 && rows_bound <= 64 && (args.defer_reduce || args.epilogue == kEpiSwiglu))
     return launch_decode(stream, args, rows_bound, cus);
-  Choice c = gemm_choice(rows_bound, args.N, args.Kp, args.defer_reduce != 0, prec == kF16,
-                         args.workspace_floats, cus);
+  Choice c = gemm_choice(rows_bound, args.N, args.Kp, args.defer_reduce != 0, prec, args.workspace_floats, cus);
   if (forced >= 0 && forced != kDecodeConfig) c = {forced, 0};
   return launch_gemm_config(stream, args, prec, rows_bound, cus, c.config, c.ksplit);
 }
