@@ -1755,12 +1755,12 @@ Choice gemm_choice(int rows, int n, uint64_t kp, bool deferred, int prec, size_t
     // 32-row tiles from 224 to 1024 rows (128-row tiles win at 2048: 1177 / 1031 us per
     // Qwen3-4B layer). Qwen3-0.6B at 96 rows against 64-row tiles: q/k/v 16.6 -> 10.6, o 15.2 -> 8.5,
     // gate+up 24.4 -> 14.6, down 16.0 -> 9.2 us; at 120 MB the two meet (q/k/v 16.0 / 16.4 us at 224
-    // rows; 157 MB of Qwen3-4B's at 65 rows 21.3 / 18.3; F32-resident, past the line at 223 rows,
-    // q/k/v 23.0 / 19.7 us and, at 65 rows, Qwen3-4B's o 26.7 / 21.8). 32-row tiles, Qwen3-4B at 512 rows:
-    // 67 -> 47, 53 -> 38, 160 -> 119, 96 -> 74 us per projection, at 224 rows 44 -> 30, 37 -> 24, 81 -> 73,
-    // 58 -> 44.
+    // rows; 157 MB of Qwen3-4B's at 65 rows 21.3 / 18.3), with F32-resident weights at 205 MB (q/k/v
+    // 19.4 / 21.9 us at 192 rows and 201 MB, 23.3 / 22.7 at 223 rows and 235 MB; Qwen3-4B's o at 65 rows and
+    // 210 MB 26.7 / 21.8). 32-row tiles, Qwen3-4B at 512 rows: 67 -> 47, 53 -> 38, 160 -> 119, 96 -> 74 us
+    // per projection, at 224 rows 44 -> 30, 37 -> 24, 81 -> 73, 58 -> 44.
     const double tile_reads = (rows + 15) / 16 * (prec == kSplitAB ? 4.0 : 2.0) * n * (double)kp;
-    if (tile_reads <= 120e6) return {0, 0};
+    if (tile_reads <= (prec == kSplitAB ? 205e6 : 120e6)) return {0, 0};
     if (rows >= 224 && rows <= 1024) return {11, deferred ? 0 : 1};
   }
   // Wide outputs of 193-223 rows: 128-row tiles, unsplit.
