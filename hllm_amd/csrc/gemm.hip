@@ -20,6 +20,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <cstdlib>
 
 namespace hllm_rocm {
@@ -1663,38 +1664,59 @@ Choice tile_choice(int rows, int n, uint64_t kp, size_t workspace_floats, int cu
   return best;
 }
 
-// Tile and K split of a many-row projection without a consumer for its partials (gate/up, LM head),
-// by the estimated time: a fixed part, the k-steps of a split times the time per k-step while no CU
-// of the fullest XCD (xcd_tile) has more than one workgroup (only_us) or at that many workgroups per
-// CU (per_us), and for a split the reduce kernel (5 us and the padded partials written and read,
-// 8 bytes each, at 4.7 TB/s). The figures are fitted to event times of every tile and split on
-// sixteen gate/up shapes (512 to 19 456 columns of K 512 to 8192) at 224 to 2048 rows; the tile
-// taken is within 4% of the best of the earlier rules' on all of them. Wide projections stay
-// unsplit (Falcon3-3B's gate+up at 1300 rows 164 us by row ranges, 143 now; Qwen3-0.6B's at 512
-// rows 32 and 17.6), narrow ones need the splits or the small tile to fill the chip: 2048 columns of K 4096 at
-// 224 rows 59 us on unsplit 128-row tiles, 23 split eight ways; K 8192 111 and 28 us; 3072
-// columns of K 2048 34.6 and 24; an LM head of 2000 features of K 2560 at 224 rows 41 and 21 us.
+// Tile and K split of a many-row projection by the estimated time: a fixed part, the k-steps of a
+// split times the time per k-step (only_us while no CU of the fullest XCD (xcd_tile) has more than
+// one workgroup; then per_us times the workgroups per CU, in whole ones, or base_us + per_us times
+// their mean number where several run beside each other), and the partials: 8 bytes per output and
+// split at 4.5 TB/s where the consumer sums them, else the reduce kernel's 5 us and the padded
+// tiles' at 4.7 TB/s. The figures are fitted to event times of every tile and split.
 struct TimedTile {
   int config, bm, most_splits, least_steps;
-  double fixed_us, only_us, per_us;
+  double fixed_us, only_us, base_us, per_us;
 };
-constexpr TimedTile kF16Tiles[] = {{12, 64, 16, 16, 8.3, 0.33, 0.275}, {9, 128, 16, 8, 10.5, 0.50, 0.40},
-                                   {15, 128, 1, 12, 11.0, 0.42, 0.51}, {18, 192, 1, 10, 14.0, 0.58, 0.69},
-                                   {16, 256, 1, 10, 15.5, 0.70, 0.87}};
+// F16 projections of 224 rows and more without a consumer for partials (gate/up, LM head), from
+// sixteen gate/up shapes (512 to 19 456 columns of K 512 to 8192) at 224 to 2048 rows; the tile
+// taken is within 4% of the best of the earlier rules' on all of them. Wide projections stay unsplit
+// (Falcon3-3B's gate+up at 1300 rows 164 us by row ranges, 143 now; Qwen3-0.6B's at 512 rows 32 and
+// 17.6), narrow ones need the splits or the small tile to fill the chip: 2048 columns of K 4096 at
+// 224 rows 59 us on unsplit 128-row tiles, 23 split eight ways; K 8192 111 and 28 us; 3072 columns
+// of K 2048 34.6 and 24; an LM head of 2000 features of K 2560 at 224 rows 41 and 21 us.
+constexpr TimedTile kF16Tiles[] = {{12, 64, 16, 16, 8.3, 0.33, 0.0, 0.275},
+                                   {9, 128, 16, 8, 10.5, 0.50, 0.0, 0.40},
+                                   {15, 128, 1, 12, 11.0, 0.42, 0.0, 0.51},
+                                   {18, 192, 1, 10, 14.0, 0.58, 0.0, 0.69},
+                                   {16, 256, 1, 10, 15.5, 0.70, 0.0, 0.87}};
+// F32 execution of 224 to 1024 rows: 32-, 64- and 128-row activation-staged tiles, with weights
+// resident as F16 and as F32, from six models' projections at 224 to 1024 rows; the tile taken is
+// within 4% of the best of the two earlier rules (64-row tiles below 384 rows and 128-row ones from
+// there; 32-row tiles throughout) on 186 of 186 and 199 of 204. Qwen3-4B's four projections, us,
+// 64- or 128-row / 32-row / now: F16-resident 384 rows 218 / 233 / 201, 512 rows 383 / 273 / 273;
+// F32-resident 384 rows 252 / 374 / 240, 512 rows 445 / 448 / 364, 1024 rows 672 / 844 / 617.
+constexpr TimedTile kSplitATiles[] = {{11, 32, 4, 8, 7.0, 0.30, 0.0, 0.26},
+                                      {12, 64, 8, 16, 11.0, 0.47, 0.0, 0.51},
+                                      {9, 128, 8, 8, 14.0, 0.86, 0.0, 0.87}};
+constexpr TimedTile kSplitABTiles[] = {{11, 32, 4, 8, 4.7, 0.505, 0.29, 0.46},
+                                       {12, 64, 8, 16, 10.2, 0.69, 0.0, 0.80},
+                                       {9, 128, 8, 8, 13.0, 1.06, 0.0, 1.20}};
 template <size_t N>
-Choice timed_choice(const TimedTile (&tiles)[N], int rows, int n, uint64_t kp, size_t workspace_floats, int cus) {
+Choice timed_choice(const TimedTile (&tiles)[N], int rows, int n, uint64_t kp, bool deferred, size_t workspace_floats,
+                    int cus) {
   const int n_tiles = (n + 255) / 256, kt = (int)(kp >> 5), per_xcd = std::max(1, cus / kXcds);
   Choice best{tiles[0].config, 1};
   double least = 1e30;
   for (const TimedTile& t : tiles) {
     const int m_tiles = (rows + t.bm - 1) / t.bm, most = std::max(1, std::min(t.most_splits, kt / t.least_steps));
-    const double partials = (double)m_tiles * t.bm * n_tiles * 256;  // per split
+    const double outputs = deferred ? (double)rows * n : (double)m_tiles * t.bm * n_tiles * 256;  // per split
     for (int want = 1, last = 0; last < most; want *= 2) {
       const int ks = last = std::min(want, most);
-      if (ks > 1 && ks * partials > (double)workspace_floats) break;
-      const int load = ((n_tiles * ks + kXcds - 1) / kXcds * m_tiles + per_xcd - 1) / per_xcd;
-      const double us = t.fixed_us + (kt + ks - 1) / ks * (load == 1 ? t.only_us : load * t.per_us) +
-                        (ks > 1 ? 5.0 + 8.0 * ks * partials / 4.7e6 : 0.0);
+      if (ks > 1 && ks * outputs > (double)workspace_floats) break;
+      const double load = (double)((n_tiles * ks + kXcds - 1) / kXcds * m_tiles) / per_xcd;
+      const double step_us = load <= 1.0         ? t.only_us
+                             : t.base_us > 0.0   ? t.base_us + t.per_us * load
+                                                 : t.per_us * std::ceil(load);
+      const double partials_us = deferred ? (ks > 1 ? 8.0 * ks : 4.0) * outputs / 4.5e6
+                                          : ks > 1 ? 5.0 + 8.0 * ks * outputs / 4.7e6 : 0.0;
+      const double us = t.fixed_us + (kt + ks - 1) / ks * step_us + partials_us;
       if (us < least) {
         least = us;
         best = {t.config, ks};
@@ -1710,7 +1732,7 @@ Choice timed_choice(const TimedTile (&tiles)[N], int rows, int n, uint64_t kp, s
 //    (gate+up, LM head) with more than 32 rows, where staging the activations in LDS once per
 //    256-feature tile wins;
 //  - F16 passes from 224 rows: tile_choice where the consumer sums the partials, else
-//    timed_choice; F32 execution by the size of the weights;
+//    timed_choice; F32 execution by the size of the weights and timed_choice;
 //  - the rest: the activation-staged kernel, BM 64, or BM 128 from 384 rows.
 // K is split while there are few output tiles. When the consumer sums the partials
 // (`deferred`) a split costs one partial write, so about 220-280 workgroups are targeted;
@@ -1722,7 +1744,7 @@ Choice gemm_choice(int rows, int n, uint64_t kp, bool deferred, int prec, size_t
   const auto rounded = [](double x) { return std::max(1, (int)(x + 0.5)); };
   if (f16 && rows >= 224)
     return deferred ? tile_choice(rows, n, kp, workspace_floats, cus)
-                    : timed_choice(kF16Tiles, rows, n, kp, workspace_floats, cus);
+                    : timed_choice(kF16Tiles, rows, n, kp, false, workspace_floats, cus);
   if (f16 && deferred && rows > 64) {
     // 65-223 rows: 64-row activation-staged tiles (at least two chunks per split), or the
     // 128-row LDS-copy tiles where they allow more than twice the K splits (less work per
@@ -1751,17 +1773,19 @@ Choice gemm_choice(int rows, int n, uint64_t kp, bool deferred, int prec, size_t
   if (!f16) {
     // F32 execution (split activations, two or three products per weight fragment): 16-row
     // register-streaming tiles while their repeated weight reads stay small (the weights, two
-    // bytes each or four resident as F32, once per 16 rows, from L2), the activation-staged kernel's
-    // 32-row tiles from 224 to 1024 rows (128-row tiles win at 2048: 1177 / 1031 us per
-    // Qwen3-4B layer). Qwen3-0.6B at 96 rows against 64-row tiles: q/k/v 16.6 -> 10.6, o 15.2 -> 8.5,
-    // gate+up 24.4 -> 14.6, down 16.0 -> 9.2 us; at 120 MB the two meet (q/k/v 16.0 / 16.4 us at 224
-    // rows; 157 MB of Qwen3-4B's at 65 rows 21.3 / 18.3), with F32-resident weights at 205 MB (q/k/v
-    // 19.4 / 21.9 us at 192 rows and 201 MB, 23.3 / 22.7 at 223 rows and 235 MB; Qwen3-4B's o at 65 rows and
-    // 210 MB 26.7 / 21.8). 32-row tiles, Qwen3-4B at 512 rows: 67 -> 47, 53 -> 38, 160 -> 119, 96 -> 74 us
-    // per projection, at 224 rows 44 -> 30, 37 -> 24, 81 -> 73, 58 -> 44.
+    // bytes each or four resident as F32, once per 16 rows, from L2), from 224 to 1024 rows
+    // timed_choice (128-row tiles win at 2048: 1177 us per Qwen3-4B layer on 32-row ones, 1031).
+    // Qwen3-0.6B at 96 rows against 64-row tiles: q/k/v 16.6 -> 10.6, o 15.2 -> 8.5, gate+up 24.4 -> 14.6,
+    // down 16.0 -> 9.2 us; at 120 MB the two meet (q/k/v 16.0 / 16.4 us at 224 rows; 157 MB of
+    // Qwen3-4B's at 65 rows 21.3 / 18.3), with F32-resident weights at 205 MB (q/k/v 19.4 / 21.9 us
+    // at 192 rows and 201 MB, 23.3 / 22.7 at 223 rows and 235 MB; Qwen3-4B's o at 65 rows and 210 MB
+    // 26.7 / 21.8) or, where the staged tiles' splits need the reduce kernel, 240 MB (gate+up of 9728
+    // columns of K 896 at 96 rows and 209 MB 20.3 / 28.1).
     const double tile_reads = (rows + 15) / 16 * (prec == kSplitAB ? 4.0 : 2.0) * n * (double)kp;
-    if (tile_reads <= (prec == kSplitAB ? 205e6 : 120e6)) return {0, 0};
-    if (rows >= 224 && rows <= 1024) return {11, deferred ? 0 : 1};
+    if (tile_reads <= (prec == kSplitA ? 120e6 : deferred ? 205e6 : 240e6)) return {0, 0};
+    if (rows >= 224 && rows <= 1024)
+      return prec == kSplitAB ? timed_choice(kSplitABTiles, rows, n, kp, deferred, workspace_floats, cus)
+                              : timed_choice(kSplitATiles, rows, n, kp, deferred, workspace_floats, cus);
   }
   // Wide outputs of 193-223 rows: 128-row tiles, unsplit.
   if (f16 && wide && !deferred && rows > 192) return {15, 1};

@@ -2,9 +2,11 @@
 weights (F16 or F32), and their results against the 64-row activation-staged tiles
 (checked against the oracle by the configuration tests).
 
-Boundary rows within 2e-5 + 2^-10 |ref|: both sides are F32 sums of 22-bit products in another order
-(2e-5 covers a layer's sums of order one over at most 8192 terms), so a value next to a rounding
-boundary moves by one F16 unit in the last place, at most 2^-10 of it."""
+Boundary rows within 5e-4 + 2^-10 |ref|. Both sides are F32 sums of 22-bit products in another order:
+the layer's F32 output (rms about 1) under any two of the 16-, 32-, 64- and 128-row tiles differs by
+1e-5 rms and 3.1e-4 at most on the largest of these shapes, because the input norm scales embedding
+rows of rms 0.02, and with them their rounding, up fifty times; the second term is the F16 unit in the
+last place by which a value next to a rounding boundary then moves."""
 import numpy as np
 import pytest
 
@@ -14,6 +16,7 @@ from tests import helpers_parity as hp
 
 pytestmark = pytest.mark.gpu
 SMALL, STAGED64 = "gemm_kernel<1, 4, 1, 1, 4, 4, ", "gemm_xlds_kernel<4, 4, 8, 4, "
+STAGED32, STAGED128 = "gemm_xlds_kernel<2, 4, 4, 4, ", "gemm_xlds_kernel<8, 4, 4, 2, "
 
 
 def tiles_and_rows(weights, hidden, intermediate, heads, rows, families):
@@ -41,7 +44,7 @@ def tiles_and_rows(weights, hidden, intermediate, heads, rows, families):
     st.close()
     error = np.abs(out[0] - out[1])
     hp.say(shape.name, weights, "rows", rows, f"max-abs {error.max():.1e}")
-    assert (error <= 2e-5 + 2.0 ** -10 * np.abs(out[1])).all(), error.max()
+    assert (error <= 5e-4 + 2.0 ** -10 * np.abs(out[1])).all(), error.max()
     return kernels
 
 
@@ -52,3 +55,16 @@ def test_tiles_by_resident_bytes(weights, rows, tile):
     kernels = tiles_and_rows(weights, 1024, 256, 16, rows, ("gemm_qkv", "gemm_o"))
     assert any(k.startswith(tile) for k in kernels["gemm_qkv"]), kernels
     assert any(k.startswith(SMALL) for k in kernels["gemm_o"]), kernels
+
+
+@pytest.mark.parametrize("weights,hidden,intermediate,heads,rows,gate_up,down", [
+    ("f32", 2560, 9728, 32, 384, STAGED128, STAGED128),   # three whole 128-row tiles
+    ("f32", 2560, 9728, 32, 1024, STAGED128, STAGED128),
+    ("f16", 2560, 9728, 32, 512, STAGED32, STAGED32),
+    ("f16", 4096, 1024, 32, 224, "gemm_reduce_kernel", ""),  # narrow and deep: a K split
+    ("f32", 4096, 1024, 32, 512, "gemm_reduce_kernel", "")])
+def test_tiles_by_estimated_time(weights, hidden, intermediate, heads, rows, gate_up, down):
+    """224 to 1024 rows: 32-row tiles alone were up to 2.3 times slower than 64- or 128-row ones."""
+    kernels = tiles_and_rows(weights, hidden, intermediate, heads, rows, ("gemm_gate_up", "gemm_down"))
+    assert any(k.startswith(gate_up) for k in kernels["gemm_gate_up"]), kernels
+    assert any(k.startswith(down) for k in kernels["gemm_down"]), kernels
