@@ -1834,12 +1834,23 @@ const DecodeShape& decode_shape(bool pair) {
   return pair ? paired : deferred;
 }
 
+bool pair_applies(const GemmArgs& a, int cus);
+
 // Whether the decode kernels run this projection: F16, and at most 64 rows where a consumer sums
 // K splits, at most 128 rows for SwiGLU (never split; measured at pair_applies) and for outputs
 // with enough features to fill the GPU unsplit (the LM head: Qwen3-4B's at 128 rows 199 -> 172 us
 // against the activation-staged kernel, 4.5 TB/s).
 bool decode_applies(const GemmArgs& a, int prec, int rows, int cus) {
   if (prec != kF16 || rows > (a.defer_reduce ? 64 : 128) || rows <= 0) return false;
+  if (a.epilogue == kEpiSwiglu && rows > 64) {
+    // A narrow gate/up of a long K has too few workgroups, and streams too long for each, once a
+    // workgroup holds more than four row tiles: there the activation-staged tiles' K splits win
+    // (pair kernel / staged, us at 65 and 128 rows, weights from HBM: 1024 columns of K 8192
+    // 37 / 24 and 42 / 26, of K 5120 26 / 22 and 29 / 23, 2048 of K 4096 21.8 / 22.0 and 24.7 / 22.9;
+    // 4096 of K 4096 22.8 / 24.4 and 25.4 / 25.6, 1024 of K 3072 17.9 / 20.7 and 20.2 / 21.2).
+    if (pair_applies(a, cus)) return a.Kp <= 3072 || (uint64_t)a.N >= a.Kp;
+    return true;
+  }
   if (a.defer_reduce || a.epilogue == kEpiSwiglu) return true;
   const DecodeShape& d = decode_shape(false);
   const int waves = d.waves >= 8 ? 8 : 4;

@@ -37,3 +37,37 @@ def test_gate_up_and_boundary_match_the_oracle(hidden, intermediate):
         hp.check_rows(oracle.f16_decode(got), oracle.f16_decode(expect), (shape.name, rows))
         st.release(seq)
     st.close()
+
+
+def gate_up_kernel(hidden, intermediate, rows):
+    """The kernel that starts gate/up of one layer, after comparing its rows with 64-row staged tiles."""
+    shape = synthetic.ModelShape(f"h{hidden}-i{intermediate}", 2, hidden, intermediate, 4, 2, 64, 300, eps=1e-6,
+                                 theta=1e4, qk_norm=False, tied=False, max_seq=128)
+    st = capi.Stage(model.stage_config(shape, 0, 1, first=True, final=False, execution="f16", kv_cache_bytes=16 << 20,
+                                       max_sequences=4, max_pass_rows=128))
+    model.synthesize(st, shape, seed=5, norm_sigma=0.1)
+    ids = np.random.default_rng(3).integers(0, shape.vocab, rows).astype(np.uint64)
+    out, kernels = [], []
+    for config in (-1, 12):
+        hp.say(shape.name, "rows", rows, "config", config)
+        seq, previous = st.allocate(rows), capi.set_gemm_config(config)
+        try:
+            st.profile("gemm_gate_up")
+            out.append(st.execute([capi.item(seq, rows, 0, sample=False)], token_ids=ids)["boundary"])
+            kernels.append([r.partition("/")[2] for r in st.profile_records() if r.startswith("gemm_gate_up/")])
+            st.profile(None)
+        finally:
+            capi.set_gemm_config(previous)
+        st.release(seq)
+    st.close()
+    hp.check_rows(oracle.f16_decode(out[0]), oracle.f16_decode(out[1]), (shape.name, rows))
+    return kernels[0]
+
+
+@pytest.mark.parametrize("hidden,intermediate,rows,kernel", [
+    (8192, 512, 64, "gemm_pair_kernel"), (8192, 512, 65, "gemm_xlds_kernel"), (4096, 1024, 128, "gemm_xlds_kernel"),
+    (4096, 2048, 128, "gemm_pair_kernel"), (3072, 256, 128, "gemm_pair_kernel")])
+def test_narrow_gate_up_of_a_long_k_above_64_rows(hidden, intermediate, rows, kernel):
+    """The pair kernel up to 128 rows only where it beats the staged tiles' K splits."""
+    kernels = gate_up_kernel(hidden, intermediate, rows)
+    assert any(k.startswith(kernel) for k in kernels), kernels
