@@ -1849,7 +1849,13 @@ bool decode_applies(const GemmArgs& a, int prec, int rows, int cus) {
     // 37 / 24 and 42 / 26, of K 5120 26 / 22 and 29 / 23, 2048 of K 4096 21.8 / 22.0 and 24.7 / 22.9;
     // 4096 of K 4096 22.8 / 24.4 and 25.4 / 25.6, 1024 of K 3072 17.9 / 20.7 and 20.2 / 21.2).
     if (pair_applies(a, cus)) return a.Kp <= 3072 || (uint64_t)a.N >= a.Kp;
-    return true;
+    // The decode kernel's 128-feature workgroups fill a CU's LDS, so more of them than CUs take a
+    // second round, and with eight row tiles it then loses on a short K (decode kernel / staged, us at 96
+    // and 128 rows: 36 864 columns of K 512 21.6 / 21.4 and 25.8 / 21.3, of K 1024 32.4 / 33.0 and
+    // 37.6 / 33.1, of K 2048 54.8 / 53.1 and 63.2 / 53.5, of K 3072 69.3 / 77.3 and 81.7 / 76.8, of K 3584
+    // 78.1 / 93.6 and 93.3 / 92.7; in one round, 32 768 columns of K 2048 36.3 / 37.3 and 38.9 / 38.1, of
+    // K 2560 37.4 / 46.4 and 41.4 / 45.8).
+    return rows <= 96 || (a.N + 127) / 128 <= cus || a.Kp > 3072;
   }
   if (a.defer_reduce || a.epilogue == kEpiSwiglu) return true;
   const DecodeShape& d = decode_shape(false);

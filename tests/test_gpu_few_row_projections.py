@@ -71,3 +71,12 @@ def test_narrow_gate_up_of_a_long_k_above_64_rows(hidden, intermediate, rows, ke
     """The pair kernel up to 128 rows only where it beats the staged tiles' K splits."""
     kernels = gate_up_kernel(hidden, intermediate, rows)
     assert any(k.startswith(kernel) for k in kernels), kernels
+
+
+@pytest.mark.parametrize("hidden,intermediate,rows,kernel", [
+    (512, 18432, 96, "gemm_decode_kernel"), (512, 18432, 97, "gemm_xlds_kernel"), (2080, 16416, 96, "gemm_decode_kernel"),
+    (2080, 16416, 128, "gemm_xlds_kernel"), (512, 16384, 128, "gemm_decode_kernel")])
+def test_wide_gate_up_of_a_short_k_above_96_rows(hidden, intermediate, rows, kernel):
+    """The decode kernel's eight row tiles only in one round of workgroups, or with a long K."""
+    kernels = gate_up_kernel(hidden, intermediate, rows)
+    assert any(k.startswith(kernel) for k in kernels), kernels
