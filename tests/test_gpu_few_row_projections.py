@@ -1,8 +1,10 @@
 """Gate/up projections of up to 128 rows (the pair kernel, and the decode kernel on wide outputs)
 and the boundary encoding that sums the last down projection's K-split partials, against the
-oracle at their edges: k-steps fewer than the waves, not a multiple of them and past one ring;
-an odd number of 32-feature groups; workgroups of one pair and of two (more pairs than CUs); 1
-to 128 rows around the 16-row tiles; row lengths that divide by four and that do not.
+oracle at their edges: k-steps fewer than the waves, not a multiple of them and past one ring of
+every row tile count (544 columns: four or five k-steps per wave of the pair kernel, three chunks of
+the decode kernel's six and eight row tiles); an odd number of 32-feature groups; workgroups of one
+pair and of two (more pairs than CUs); 1 to 128 rows around the 16-row tiles; row lengths that divide
+by four and that do not, both with partials for the boundary (66 columns from 1600: five).
 
 A one-layer first stage returns its boundary rows. Bounds per row as for the other F16 slices
 (max-abs 2e-2, cosine 0.9999)."""
@@ -18,7 +20,8 @@ pytestmark = pytest.mark.gpu
 ROWS = (1, 15, 16, 17, 31, 33, 48, 49, 64, 65, 81, 96, 97, 128)
 
 
-@pytest.mark.parametrize("hidden,intermediate", [(64, 32), (66, 96), (96, 160), (160, 4128), (544, 288), (64, 8224)])
+@pytest.mark.parametrize("hidden,intermediate", [(64, 32), (66, 96), (96, 160), (160, 4128), (544, 288), (64, 8224),
+                                                 (66, 1600), (544, 4128), (544, 8224)])
 def test_gate_up_and_boundary_match_the_oracle(hidden, intermediate):
     shape = synthetic.ModelShape(f"h{hidden}-i{intermediate}", 2, hidden, intermediate, 4, 2, 64, 300, eps=1e-6,
                                  theta=1e4, qk_norm=False, tied=False, max_seq=128)

@@ -1,6 +1,7 @@
 """The LM head of 65 to 128 sampled rows (the decode GEMM's eight row tiles, unsplit): logits and the five
 best log-probabilities against the oracle, and the fused greedy token against the first maximum
-of the logits. Vocabulary just wide enough for that kernel and not a multiple of its tiles.
+of the logits. Vocabulary just wide enough for that kernel and not a multiple of its tiles; hidden
+sizes whose 128 rows fit in LDS whole (up to 576) and whose chunks of four k-steps are staged in turn.
 
 Logits within max-abs 2e-2 and cosine 0.9999 (F16 slices); log-probabilities against the
 64-bit log-softmax of the GPU's own logits to 1e-12 (a few roundings of 64-bit sums)."""
@@ -13,23 +14,24 @@ from tests import helpers_parity as hp
 from tests import models
 
 pytestmark = pytest.mark.gpu
-SHAPE = synthetic.ModelShape("head-rows", 1, 96, 64, 4, 2, 64, 16500, eps=1e-6, theta=1e4, qk_norm=False, tied=False,
-                             max_seq=128)
 
 
-def test_head_of_65_to_128_rows():
-    st = capi.Stage(model.stage_config(SHAPE, execution="f16", kv_cache_bytes=16 << 20, max_sequences=128,
+@pytest.mark.parametrize("hidden", [96, 608])
+def test_head_of_65_to_128_rows(hidden):
+    shape = synthetic.ModelShape(f"head-rows-h{hidden}", 1, hidden, 64, 4, 2, 64, 16500, eps=1e-6, theta=1e4, qk_norm=False,
+                                 tied=False, max_seq=128)
+    st = capi.Stage(model.stage_config(shape, execution="f16", kv_cache_bytes=16 << 20, max_sequences=128,
                                        max_pass_rows=128))
-    model.synthesize(st, SHAPE, seed=5, norm_sigma=0.1)
-    ost = oracle.OracleStage(models.synthetic_stage(SHAPE, seed=5, norm_sigma=0.1))
-    ids = np.random.default_rng(3).integers(0, SHAPE.vocab, 128).astype(np.uint64)
+    model.synthesize(st, shape, seed=5, norm_sigma=0.1)
+    ost = oracle.OracleStage(models.synthetic_stage(shape, seed=5, norm_sigma=0.1))
+    ids = np.random.default_rng(3).integers(0, shape.vocab, 128).astype(np.uint64)
     expect = []
     for i in ids:
         trace = []
         ost.execute(np.array([i], np.uint64), 0, ost.allocate_sequence(1), trace)
         expect.append(trace[-1])
     for rows in (64, 65, 113, 128):
-        hp.say(SHAPE.name, "rows", rows)
+        hp.say(shape.name, "rows", rows)
 
         def run(**options):
             seqs = [st.allocate(1) for _ in range(rows)]
