@@ -1641,9 +1641,14 @@ Choice tile_choice(int rows, int n, uint64_t kp, size_t workspace_floats, int cu
                              {9, 128, 2, 0.80, 1.00}};
   const int n_tiles = (n + 255) / 256, kt = (int)(kp >> 5);
   const double partial_us = 8.0 * rows * n / 4.5e6;
-  // Above 1536 rows (there the row tiles alone fill the CUs on most shapes) the K split is that
-  // of 280 workgroups of 128-row tiles, as for F32 execution: full passes of long prompts keep
-  // their order of summation, and with it the tokens at near ties, whatever tile runs them.
+  // Above 1536 rows the K split is that of about 280 workgroups of 128-row tiles, the earlier choice
+  // for such passes, although free splits are faster (Qwen3-4B at 2048 rows o 66 -> 50 us, down 134 ->
+  // 98): another order of summation in the full passes that prefill long prompts turned one or two
+  // near-tied greedy tokens in 64 of a whole served model, more than perf/cases.py allows it
+  // (serve_64). Passes of 224 to 1536 rows carry no such bound. The sums keep the earlier order only
+  // where both tiles cut K alike: the LDS-copy tiles split at ceil(KT / splits) k-steps and take at
+  // most KT / 12 (or / 10) splits, the activation-staged tiles round a split up to four k-steps and
+  // take at most KT / 8 (Qwen3-4B's projections are alike on both, Qwen3-0.6B's o at 1600 rows is not).
   const int kept = rows > 1536 ? deferred_splits(rows, n, kt) : 0;
   Choice best{15, 1};
   double least = 1e30;
@@ -1728,9 +1733,10 @@ Choice timed_choice(const TimedTile (&tiles)[N], int rows, int n, uint64_t kp, b
 
 // Projection configuration by pass rows and shape, from sweeps of the Qwen3 projection
 // shapes on MI355X with weights streamed from HBM:
-//  - up to 64 rows: the register-streaming kernels (BM 16/32/64), except for very wide outputs
-//    (gate+up, LM head) with more than 32 rows, where staging the activations in LDS once per
-//    256-feature tile wins;
+//  - up to 64 rows (F32 execution, and F16 projections that the decode kernels leave, such as an LM
+//    head over a small vocabulary): the register-streaming kernels (BM 16/32/64), except for very
+//    wide outputs (gate+up, LM head) with more than 32 rows, where staging the activations in LDS
+//    once per 256-feature tile wins;
 //  - F16 passes from 224 rows: tile_choice where the consumer sums the partials, else
 //    timed_choice; F32 execution by the size of the weights and timed_choice;
 //  - the rest: the activation-staged kernel, BM 64, or BM 128 from 384 rows.
