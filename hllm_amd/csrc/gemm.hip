@@ -1793,8 +1793,11 @@ Choice gemm_choice(int rows, int n, uint64_t kp, bool deferred, int prec, size_t
       return prec == kSplitAB ? timed_choice(kSplitABTiles, rows, n, kp, deferred, workspace_floats, cus)
                               : timed_choice(kSplitATiles, rows, n, kp, deferred, workspace_floats, cus);
   }
-  // Wide outputs of 193-223 rows: 128-row tiles, unsplit.
-  if (f16 && wide && !deferred && rows > 192) return {15, 1};
+  // Wide outputs of 193-223 rows: 128-row tiles, unsplit (F32 execution: unless two splits of them fit
+  // the CUs at once; an LM head of 16 500 features at 223 rows, 130 tiles, F16-resident of K 1024 41 us
+  // unsplit, 66 in two rounds of splits and a reduce kernel, F32-resident of K 2560 99 and 126; gate+up
+  // of 16 384 columns of K 2048, 128 tiles, F32-resident 83 and 68).
+  if (wide && !deferred && rows > 192 && rows < 224 && (f16 || (n + 255) / 256 * 4 > cus)) return {f16 ? 15 : 9, 1};
   const int bm = rows >= 384 || (wide && rows > 192) ? 128 : 64;
   const int config = bm == 128 ? 9 : 12;
   const int kc = bm == 128 ? 4 : 8;

@@ -68,3 +68,32 @@ def test_tiles_by_estimated_time(weights, hidden, intermediate, heads, rows, gat
     kernels = tiles_and_rows(weights, hidden, intermediate, heads, rows, ("gemm_gate_up", "gemm_down"))
     assert any(k.startswith(gate_up) for k in kernels["gemm_gate_up"]), kernels
     assert any(k.startswith(down) for k in kernels["gemm_down"]), kernels
+
+
+@pytest.mark.parametrize("weights", ["f16", "f32"])
+def test_wide_head_of_193_to_223_rows_is_not_split(weights):
+    """130 tiles of 128 rows: splits of them would take a second round of workgroups."""
+    shape = synthetic.ModelShape("v16500", 1, 1024, 64, 4, 2, 64, 16500, eps=1e-6, theta=1e4, qk_norm=False, tied=False,
+                                 max_seq=64)
+    st = capi.Stage(model.stage_config(shape, execution="f32", weights=weights, kv_cache_bytes=64 << 20,
+                                       max_sequences=223, max_pass_rows=256))
+    model.synthesize(st, shape, seed=5, norm_sigma=0.1)
+    ids = np.random.default_rng(3).integers(0, shape.vocab, 223).astype(np.uint64)
+    logits = []
+    for config in (-1, 12):
+        hp.say(shape.name, weights, "config", config)
+        seqs, previous = [st.allocate(1) for _ in ids], capi.set_gemm_config(config)
+        try:
+            st.profile("gemm_lm_head")
+            logits.append(st.execute([capi.item(s, 1, 0) for s in seqs], token_ids=ids, want_logits=True)["logits"])
+            kernels = [r.partition("/")[2] for r in st.profile_records() if r.startswith("gemm_lm_head/")]
+            st.profile(None)
+        finally:
+            capi.set_gemm_config(previous)
+        for s in seqs:
+            st.release(s)
+        if config < 0:
+            assert len(kernels) == 1 and kernels[0].startswith(STAGED128), kernels
+    st.close()
+    # F32 logits, the suite's bound for another order of summation.
+    assert (np.abs(logits[0] - logits[1]) <= 2e-4 + 1e-4 * np.abs(logits[1])).all()
