@@ -1786,9 +1786,10 @@ Choice gemm_choice(int rows, int n, uint64_t kp, bool deferred, int prec, size_t
     // Qwen3-4B's at 65 rows 21.3 / 18.3), with F32-resident weights at 205 MB (q/k/v 19.4 / 21.9 us
     // at 192 rows and 201 MB, 23.3 / 22.7 at 223 rows and 235 MB; Qwen3-4B's o at 65 rows and 210 MB
     // 26.7 / 21.8) or, where the staged tiles' splits need the reduce kernel, 240 MB (gate+up of 9728
-    // columns of K 896 at 96 rows and 209 MB 20.3 / 28.1).
+    // columns of K 896 at 96 rows and 209 MB 20.3 / 28.1), but not on wide outputs, whose weights the
+    // row tiles read from beyond L2 each time (LM head of 16 500 features of K 1024 at 33 rows 36.3 / 28.9).
     const double tile_reads = (rows + 15) / 16 * (prec == kSplitAB ? 4.0 : 2.0) * n * (double)kp;
-    if (tile_reads <= (prec == kSplitA ? 120e6 : deferred ? 205e6 : 240e6)) return {0, 0};
+    if (tile_reads <= (prec == kSplitA ? 120e6 : deferred ? 205e6 : wide ? 0.0 : 240e6)) return {0, 0};
     if (rows >= 224 && rows <= 1024)
       return prec == kSplitAB ? timed_choice(kSplitABTiles, rows, n, kp, deferred, workspace_floats, cus)
                               : timed_choice(kSplitATiles, rows, n, kp, deferred, workspace_floats, cus);
